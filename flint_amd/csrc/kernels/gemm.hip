@@ -835,6 +835,10 @@ hipError_t gemm_tn_workspace(size_t m, size_t n, size_t k, size_t* bytes) {
 
 hipError_t launch_gemm_nt(void* y, const void* x, const void* w, const void* bias, void* aux,
                           Epilogue e, size_t m, size_t n, size_t k, hipStream_t stream) {
+    SmallPlan small;
+    if (gemm_small_plan(GemmLayout::kNT, e, 1, m, n, k, 1, &small))
+        return launch_gemm_small(small, GemmLayout::kNT, e, y, x, w, bias, aux, 1.0f, 1, m, n, k,
+                                 false, nullptr, stream);
     if (gemm_pipe_eligible(GemmLayout::kNT, e, m, n, k))
         return launch_gemm_pipe(GemmLayout::kNT, e, y, x, w, bias, aux, 1.0f, 1, m, n, k, false,
                                 nullptr, 0, stream);
@@ -852,6 +856,10 @@ hipError_t launch_gemm_nt(void* y, const void* x, const void* w, const void* bia
 
 hipError_t launch_gemm_nn(void* y, const void* x, const void* w, const void* aux, Epilogue e,
                           size_t m, size_t n, size_t k, hipStream_t stream) {
+    SmallPlan small;
+    if (gemm_small_plan(GemmLayout::kNN, e, 1, m, n, k, 1, &small))
+        return launch_gemm_small(small, GemmLayout::kNN, e, y, x, w, nullptr, const_cast<void*>(aux),
+                                 1.0f, 1, m, n, k, false, nullptr, stream);
     if (gemm_pipe_eligible(GemmLayout::kNN, e, m, n, k))
         return launch_gemm_pipe(GemmLayout::kNN, e, y, x, w, nullptr, const_cast<void*>(aux), 1.0f,
                                 1, m, n, k, false, nullptr, 0, stream);
@@ -873,7 +881,14 @@ hipError_t launch_gemm_tn_split(void* y, const void* x, const void* w, size_t m,
     op.accumulate = accumulate ? 1 : 0;
     op.partials = splits > 1 ? static_cast<float*>(workspace) : nullptr;
     hipError_t err;
-    if (gemm_pipe_eligible(GemmLayout::kTN, kTnFloat, m, n, k)) {
+    SmallPlan small;
+    if (gemm_small_plan(GemmLayout::kTN, kTnFloat, 1, m, n, k, op.partials != nullptr ? splits : 1,
+                        &small)) {
+        // Its own split count, at most the plan's, like the pipeline.
+        splits = small.splits;
+        err = launch_gemm_small(small, GemmLayout::kTN, kTnFloat, y, x, w, nullptr, nullptr, 1.0f, 1,
+                                m, n, k, accumulate, splits > 1 ? op.partials : nullptr, stream);
+    } else if (gemm_pipe_eligible(GemmLayout::kTN, kTnFloat, m, n, k)) {
         // The pipeline picks its own split count, at most the plan's.
         int used = 1;
         err = launch_gemm_pipe_tn(y, x, w, m, n, k, accumulate, op.partials, splits, &used, stream);
@@ -908,6 +923,11 @@ hipError_t launch_gemm_tn(void* y, const void* x, const void* w, size_t m, size_
 hipError_t launch_gemm_nt_batched(void* y, const void* x, const void* w, size_t batches,
                                   size_t m, size_t n, size_t k, float scale, hipStream_t stream,
                                   bool causal) {
+    SmallPlan small;
+    if (gemm_small_plan(GemmLayout::kNT, Epilogue::kScale, batches, m, n, k, 1, &small))
+        return launch_gemm_small(small, GemmLayout::kNT, Epilogue::kScale, y, x, w, nullptr, nullptr,
+                                 scale, batches, m, n, k, false, nullptr, stream,
+                                 causal && m == n);
     if (gemm_pipe_eligible(GemmLayout::kNT, Epilogue::kScale, m, n, k))
         return launch_gemm_pipe(GemmLayout::kNT, Epilogue::kScale, y, x, w, nullptr, nullptr, scale,
                                 batches, m, n, k, false, nullptr, 0, stream, causal && m == n);
@@ -923,6 +943,11 @@ bool gemm_batched_causal_taken(GemmLayout l, size_t m, size_t n, size_t k) {
 
 hipError_t launch_gemm_nn_batched(void* y, const void* x, const void* w, size_t batches,
                                   size_t m, size_t n, size_t k, hipStream_t stream, bool causal) {
+    SmallPlan small;
+    if (gemm_small_plan(GemmLayout::kNN, Epilogue::kNone, batches, m, n, k, 1, &small))
+        return launch_gemm_small(small, GemmLayout::kNN, Epilogue::kNone, y, x, w, nullptr, nullptr,
+                                 1.0f, batches, m, n, k, false, nullptr, stream,
+                                 causal && m == k);
     if (gemm_pipe_eligible(GemmLayout::kNN, Epilogue::kNone, m, n, k))
         return launch_gemm_pipe(GemmLayout::kNN, Epilogue::kNone, y, x, w, nullptr, nullptr, 1.0f,
                                 batches, m, n, k, false, nullptr, 0, stream, causal && m == k);
@@ -934,6 +959,11 @@ hipError_t launch_gemm_nn_batched_views(void* y, const void* x, const void* w, s
                                         size_t m, size_t n, size_t k, const HeadView& wv,
                                         const HeadView& yv, hipStream_t stream, bool causal) {
     if (!gemm_pipe_eligible(GemmLayout::kNN, Epilogue::kNone, m, n, k)) return hipErrorInvalidValue;
+    SmallPlan small;
+    if (gemm_small_plan(GemmLayout::kNN, Epilogue::kNone, batches, m, n, k, 1, &small))
+        return launch_gemm_small(small, GemmLayout::kNN, Epilogue::kNone, y, x, w, nullptr, nullptr,
+                                 1.0f, batches, m, n, k, false, nullptr, stream,
+                                 causal && m == k, &wv, &yv);
     return launch_gemm_pipe(GemmLayout::kNN, Epilogue::kNone, y, x, w, nullptr, nullptr, 1.0f,
                             batches, m, n, k, false, nullptr, 0, stream, causal && m == k, &wv,
                             &yv);
@@ -943,6 +973,11 @@ hipError_t launch_gemm_tn_batched_views(void* y, const void* x, const void* w, s
                                         size_t m, size_t n, size_t k, const HeadView& wv,
                                         const HeadView& yv, hipStream_t stream, bool causal) {
     if (!gemm_pipe_eligible(GemmLayout::kTN, Epilogue::kNone, m, n, k)) return hipErrorInvalidValue;
+    SmallPlan small;
+    if (gemm_small_plan(GemmLayout::kTN, Epilogue::kNone, batches, m, n, k, 1, &small))
+        return launch_gemm_small(small, GemmLayout::kTN, Epilogue::kNone, y, x, w, nullptr, nullptr,
+                                 1.0f, batches, m, n, k, false, nullptr, stream,
+                                 causal && m == k, &wv, &yv);
     return launch_gemm_pipe(GemmLayout::kTN, Epilogue::kNone, y, x, w, nullptr, nullptr, 1.0f,
                             batches, m, n, k, false, nullptr, 0, stream, causal && m == k, &wv,
                             &yv);
@@ -950,6 +985,11 @@ hipError_t launch_gemm_tn_batched_views(void* y, const void* x, const void* w, s
 
 hipError_t launch_gemm_tn_batched(void* y, const void* x, const void* w, size_t batches,
                                   size_t m, size_t n, size_t k, hipStream_t stream, bool causal) {
+    SmallPlan small;
+    if (gemm_small_plan(GemmLayout::kTN, Epilogue::kNone, batches, m, n, k, 1, &small))
+        return launch_gemm_small(small, GemmLayout::kTN, Epilogue::kNone, y, x, w, nullptr, nullptr,
+                                 1.0f, batches, m, n, k, false, nullptr, stream,
+                                 causal && m == k);
     if (gemm_pipe_eligible(GemmLayout::kTN, Epilogue::kNone, m, n, k))
         return launch_gemm_pipe(GemmLayout::kTN, Epilogue::kNone, y, x, w, nullptr, nullptr, 1.0f,
                                 batches, m, n, k, false, nullptr, 0, stream, causal && m == k);

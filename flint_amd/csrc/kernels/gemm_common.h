@@ -17,8 +17,36 @@ typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
 typedef _Float16 f16x4 __attribute__((ext_vector_type(4)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
+typedef int i32x4 __attribute__((ext_vector_type(4)));
+typedef int i32x2 __attribute__((ext_vector_type(2)));
 typedef __attribute__((address_space(3))) _Float16 lds_half;
 
+// The two 4-half results of a pair of ds_read_b64_tr_b16, k 0..3 and 4..7.
+struct TrFrag {
+    i32x2 lo, hi;
+};
+__device__ __forceinline__ f16x8 as_f16x8(const f16x8& v) { return v; }
+__device__ __forceinline__ f16x8 as_f16x8(const TrFrag& f) {
+    return __builtin_shufflevector(__builtin_bit_cast(f16x4, f.lo), __builtin_bit_cast(f16x4, f.hi), 0,
+                                   1, 2, 3, 4, 5, 6, 7);
+}
+
+// Key of the [rows][BK] layouts, XORed into a row's 16-byte chunk index. The
+// 16 lanes a ds_read_b128 serves per cycle read one chunk of 16 consecutive
+// rows, which must land on 16 distinct 16-byte bank groups (64 banks):
+//  * BK = 32 (64-byte rows, 4 chunks): rows r, r + 4, r + 8, r + 12 share
+//    bank groups before the XOR; ((row >> 1) ^ (row >> 2)) & 3 tells them apart.
+//  * BK = 64 (128-byte rows, 8 chunks): the 8 even (odd) rows share 8 bank
+//    groups; (row >> 1) & 7 gives each its own.
+template <int BK>
+__device__ __forceinline__ int row_key(int row) {
+    if constexpr (BK == 32) return ((row >> 1) ^ (row >> 2)) & 3;
+    else return (row >> 1) & 7;
+}
+// Key of the [32 k][rows] layout: rows k .. k + 3, which one transposing read
+// of 16 lanes touches (2 chunks each), land on 8 distinct chunk positions of an
+// aligned group of 8 (the XOR stays inside the group, hence inside the row).
+__host__ __device__ constexpr int kmajor_key(int k) { return 2 * (k & 3); }
 
 enum class Layout { kNT, kNN, kTN };
 // What the kernel's store stage does. kTn writes FP32 (plain, accumulate or a

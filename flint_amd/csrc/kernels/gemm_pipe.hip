@@ -1,7 +1,7 @@
 // The GEMM pipeline on gfx950 with one wave per SIMD and large wave tiles,
 // for all three layouts (NT, NN, TN, and their batched forms) whenever k is a
-// multiple of 32 and the output rows are 16-byte multiples. Other shapes run
-// gemm.hip's kernels.
+// multiple of 32 and the output rows are 16-byte multiples. Products of few
+// tiles run gemm_small.hip's kernels, other shapes gemm.hip's.
 //
 // Why this shape of kernel (measured on MI355X):
 //  * A CU's L2 -> LDS rate depends on the row piece one load covers: 64-byte
@@ -65,20 +65,7 @@ namespace {
 
 constexpr int kPipeBK = 32;
 
-typedef int i32x4 __attribute__((ext_vector_type(4)));
-typedef int i32x2 __attribute__((ext_vector_type(2)));
-
 constexpr int cap63(int n) { return n < 63 ? n : 63; }
-
-// The two 4-half results of a pair of ds_read_b64_tr_b16, k 0..3 and 4..7.
-struct TrFrag {
-    i32x2 lo, hi;
-};
-__device__ __forceinline__ f16x8 as_f16x8(const f16x8& v) { return v; }
-__device__ __forceinline__ f16x8 as_f16x8(const TrFrag& f) {
-    return __builtin_shufflevector(__builtin_bit_cast(f16x4, f.lo), __builtin_bit_cast(f16x4, f.hi), 0,
-                                   1, 2, 3, 4, 5, 6, 7);
-}
 
 // Cache policy of the epilogue's stores: non-temporal (the nt bit). Outputs
 // are written once and read by a later kernel, not by this one; marked as
@@ -92,23 +79,6 @@ __device__ __forceinline__ void wait_vm_lgkm0() {
     static_assert(N >= 0 && N < 64, "vmcnt range");
     __builtin_amdgcn_s_waitcnt((N & 15) | ((N >> 4) << 14) | (7 << 4));
 }
-
-// Key of the [rows][BK] layouts, XORed into a row's 16-byte chunk index. The
-// 16 lanes a ds_read_b128 serves per cycle read one chunk of 16 consecutive
-// rows, which must land on 16 distinct 16-byte bank groups (64 banks):
-//  * BK = 32 (64-byte rows, 4 chunks): rows r, r + 4, r + 8, r + 12 share
-//    bank groups before the XOR; ((row >> 1) ^ (row >> 2)) & 3 tells them apart.
-//  * BK = 64 (128-byte rows, 8 chunks): the 8 even (odd) rows share 8 bank
-//    groups; (row >> 1) & 7 gives each its own.
-template <int BK>
-__device__ __forceinline__ int row_key(int row) {
-    if constexpr (BK == 32) return ((row >> 1) ^ (row >> 2)) & 3;
-    else return (row >> 1) & 7;
-}
-// Key of the [32 k][rows] layout: rows k .. k + 3, which one transposing read
-// of 16 lanes touches (2 chunks each), land on 8 distinct chunk positions of an
-// aligned group of 8 (the XOR stays inside the group, hence inside the row).
-__host__ __device__ constexpr int kmajor_key(int k) { return 2 * (k & 3); }
 
 // Waves of a workgroup along n: 2 x 2 waves, or 4 x 1 for 64-wide tiles.
 __host__ __device__ constexpr int pipe_waves_n(int bn) { return bn >= 128 ? 2 : 1; }
@@ -1305,6 +1275,35 @@ bool gemm_pipe_eligible(GemmLayout gl, Epilogue e, size_t m, size_t n, size_t k)
         return false;
     }
     return true;
+}
+
+// Per k-step of 64 a tile takes about 1 us * area / 256^2 / pipe_eff; a
+// round's prologue and epilogue 1.5 us, TN's FP32 output 4 (measured on
+// one-round products: NT 256 x 3072 x 768 6.6 us past its launch, 24 x 256 x
+// 256 x 64 2.0, TN 768 x 768 x 64 4.5 and x 256 5.8).
+double gemm_pipe_estimate(GemmLayout gl, Epilogue e, size_t slices, size_t m, size_t n, size_t k,
+                          int max_splits) {
+    constexpr double kInfinite = 1e300;
+    int cus = 256;
+    if (!gemm_pipe_eligible(gl, e, m, n, k) || device_cus(&cus) != hipSuccess) return kInfinite;
+    const Layout l = layout_of(gl);
+    const Store st = store_of(e, l);
+    PipeConfig c;
+    int sp = 1;
+    if (e == kTnFloat) plan_tn(m, n, k, max_splits, cus, false, nullptr, &c, &sp);
+    else c = pick_pipe(m, n, k, slices, cus, st, l);
+    const double tiles = double((m + c.bm - 1) / c.bm) * double((n + c.bn - 1) / c.bn) *
+                         double(slices) * sp;
+    const double rounds = std::ceil(tiles / cus);
+    const double steps = double(k) / sp / 64.0;
+    // 32-deep steps of row-major operands load half lines, at half the rate
+    // while few tiles are in flight (NN 3000 x 744 x 2976 56 us in one round).
+    const bool half_lines = c.bk == 32 && l != Layout::kTN;
+    const double step_us = double(c.bm) * double(c.bn) / 65536.0 / pipe_eff(c, st, l) *
+                           (l == Layout::kNN ? 1.1 : 1.0) * (half_lines ? 2.0 : 1.0);
+    double us = rounds * (steps * step_us + (l == Layout::kTN ? 4.0 : 1.5));
+    if (sp > 1) us += 3.0 + double(sp + 2) * double(m) * double(n) * 4.0 / 5e6;
+    return us;
 }
 
 hipError_t launch_gemm_pipe(GemmLayout gl, Epilogue e, void* y, const void* x, const void* w,

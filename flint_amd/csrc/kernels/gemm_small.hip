@@ -1,0 +1,636 @@
+// GEMMs whose output has few tiles: 64 x 64 and 32 x 32 tiles, one per
+// workgroup, for every layout, epilogue and size the entry points take.
+//
+// A product with a few hundred rows leaves gemm_pipe.hip's 128 x 192 tiles on
+// 4 to 48 of the 256 CUs, and each of those then streams its whole k-range at
+// one CU's load rate. What bounds such a product is the bytes that one CU has
+// to stream (its tile's two operand strips) and the latency of the first of
+// them, so the tile here is as small as the MFMA's 32 x 32 allows:
+//  * 256 threads. WM x WN of the four waves each own one 32 x 32 block; all
+//    four issue the operand loads (a CU's load rate grows with the waves that
+//    issue: one wave alone reached a quarter of it), so a 32 x 32 tile has one
+//    MFMA wave and three that only load.
+//  * k-steps of 64 through S LDS stages by direct-to-LDS buffer loads, S steps
+//    in flight, one barrier a step. The fragments of step s + 1 are read
+//    while step s's MFMAs run, which also frees step s's stage for the load
+//    of step s + S at the same barrier.
+//  * Each 32 x 32 block is one chain of v_mfma_f32_32x32x16_f16 over k in
+//    ascending order from a zero accumulator, as in the other GEMM kernels:
+//    the same sums, bit for bit, whichever kernel a shape runs on.
+//  * The epilogue's inputs (bias, residual, pre, the old y) load before the
+//    k-loop; the sums go through LDS once so that every thread finishes 4 or 8
+//    consecutive columns of a row.
+//  * Ragged sizes: rows and columns past the operands read zeros or values
+//    that only reach outputs that are not stored; a k tail (k % 64) reads
+//    zeros from both operands.
+//  * Larger tiles (32 x 64 to 128 x 64, up to eight waves) take over as the
+//    tile count passes the CUs, until gemm_pipe.hip's tiles fill the GPU:
+//    gemm_small_plan compares both by their estimated times.
+// Measured (one MI355X, operands rotated past the caches, launch included,
+// before -> after): NT 64 x 768 x 3072 22.5 -> 9.4 us, 256 x 768 x 768 9.6 ->
+// 4.6, 1024 x 768 x 3072 25 -> 12.9; NN 256 x 768 x 50304 518 -> 178; TN 768 x
+// 768 x 256 9.1 -> 4.8; ragged NT 1000 x 200 x 800 14.0 -> 5.0, TN 768 x 768 x
+// 1000 60 -> 8.0. A tile's k-step takes 0.14 to 0.3 us: at 32 x 32 four
+// dependent MFMAs (about 150 cycles) and a barrier every second step, at 64 x
+// 64 the 32 KB of fragment reads (about 110 B a cycle).
+#include <hip/hip_runtime.h>
+
+#include <algorithm>
+#include <cstdio>
+#include <type_traits>
+
+#include "common/common.h"
+#include "common/tuning.h"
+#include "kernels/gemm_common.h"
+#include "kernels/kernels.h"
+
+namespace flint {
+namespace {
+
+constexpr int kStep = 64;   // k per step
+
+// gemm_pipe_estimate's value for a shape the pipeline does not take.
+constexpr double kNoEstimate = 1e300;
+
+// A split TN's sum of its partials: a launch of its own (us).
+constexpr double kSplitSumUs = 3.0;
+
+// A buffer offset past every resource: the load returns zeros.
+constexpr unsigned kOutside = 0xfffffff0u;
+
+// The FP32 value itself, however it was formed: a conversion that follows
+// rounds it and not the exact product behind it.
+__device__ __forceinline__ float settled(float x) {
+    asm("" : "+v"(x));
+    return x;
+}
+
+template <int WM, int WN, int NW, int S, int U, Layout L, Store ST, bool HV = false>
+__global__ void __launch_bounds__(NW * 64) gemm_small(Operands op, TileArgs ta) {
+    // The host pass only needs a kernel to emit a launch stub for.
+#if defined(__HIP_DEVICE_COMPILE__)
+    static_assert(WM * WN <= NW, "at most one block per wave");
+    static_assert(S % U == 0 && S / U >= 2, "a group in use, one landing");
+    constexpr int T = NW * 64;
+    constexpr int BM = 32 * WM, BN = 32 * WN;
+    // x (rows m, the MFMA's B operand) and w (rows n, its A operand) are
+    // k-major ([64 k][rows] in LDS) or row-major ([rows][64 k]).
+    constexpr bool kXM = L == Layout::kTN;
+    constexpr bool kWM = L != Layout::kNT;
+    using XFrag = std::conditional_t<kXM, TrFrag, f16x8>;
+    using WFrag = std::conditional_t<kWM, TrFrag, f16x8>;
+    constexpr bool kBias =
+        ST == Store::kBias || ST == Store::kBiasGelu || ST == Store::kBiasResidual;
+    constexpr bool kF32 = ST == Store::kBiasResidual || ST == Store::kTn;
+    // A step's 1 KB loads, x's first, dealt to the waves in turn.
+    constexpr int kLoadsA = BM / 8, kLoads = (BM + BN) / 8, PER = kLoads / NW;
+    static_assert(kLoads % NW == 0 && S * PER < 64, "whole loads per wave, vmcnt range");
+    constexpr int kGroupLoads = U * PER;
+    constexpr int kStage = (BM + BN) * kStep;
+    constexpr int kLd = BN + 4;                       // staged sums: floats a row
+    static_assert(BM * kLd * 2 <= S * kStage, "the sums reuse the stages");
+    __shared__ __attribute__((aligned(16))) _Float16 lds[S * kStage];
+
+    const int tid = threadIdx.x;
+    const int lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int m = op.m, n = op.n, K = op.k;
+    const bool split = ST == Store::kTn && op.partials != nullptr;
+
+    // ---- this workgroup's tile
+    int slice, tm, tn;
+    if (op.causal && L != Layout::kNT) {
+        // A tile's k-range grows (NN) or shrinks (TN) with its row block:
+        // longest first.
+        const unsigned per_row = unsigned(ta.slices) * unsigned(ta.tiles_n);
+        const int d = int(blockIdx.x / per_row);
+        const unsigned rem = blockIdx.x % per_row;
+        tm = L == Layout::kNN ? ta.tiles_m - 1 - d : d;
+        slice = int(rem / unsigned(ta.tiles_n));
+        tn = int(rem % unsigned(ta.tiles_n));
+    } else {
+        map_tile(ta, blockIdx.x, &slice, &tm, &tn);
+    }
+    const int m0 = tm * BM, n0 = tn * BN;
+    if (L == Layout::kNT && op.causal && n0 >= m0 + BM) return;   // above the diagonal
+    int k_begin = 0, k_end = K;
+    if (L == Layout::kNN && op.causal) k_end = min(K, (m0 + BM + kStep - 1) / kStep * kStep);
+    if (L == Layout::kTN && op.causal) k_begin = m0 / kStep * kStep;
+    const _Float16* xs = op.x;
+    const _Float16* ws = op.w;
+    size_t y_off = 0;
+    if (split) {
+        k_begin = slice * ta.split_len;
+        k_end = min(K, k_begin + ta.split_len);
+        y_off = size_t(slice) * m * n;
+    } else if (ta.slices > 1) {
+        xs += size_t(slice) * m * K;
+        ws += HV ? head_view_offset(op.wv, slice) : size_t(slice) * n * K;
+        y_off = HV ? head_view_offset(op.yv, slice) : size_t(slice) * m * n;
+    }
+    const int a_ld = kXM ? m : K;
+    const int b_ld = kWM ? (HV ? op.wv.ld : n) : K;
+    const size_t y_ld = HV ? op.yv.ld : n;
+
+    // ---- operand loads. Row-major: a resource over the tile's valid rows,
+    // the k-step in the scalar offset, chunks past k_end sent outside.
+    // k-major: a resource from the step's first k row to the operand's end.
+    const _Float16* const a = kXM ? xs + m0 : xs + size_t(m0) * K;
+    const _Float16* const b = kWM ? ws + n0 : ws + size_t(n0) * K;
+    const size_t a_bytes = kXM ? (size_t(K) * m - m0) * 2 : size_t(min(BM, m - m0)) * K * 2;
+    const size_t b_bytes = kWM ? (size_t(K - 1) * b_ld + n - n0) * 2
+                               : size_t(min(BN, n - n0)) * K * 2;
+    // Load v = q NW + wave of a step fills LDS bytes [v KB, v KB + 1 KB) of its
+    // stage (x's region, then w's); lane l writes bytes 16 l .. + 15 of it.
+    unsigned voff[PER];
+    int kofs[PER];   // row-major: the lane's k within a step
+    auto of_x = [&](int q) {
+        return kLoadsA % NW == 0 ? q < kLoadsA / NW : q * NW + wave < kLoadsA;
+    };
+    auto place = [&](int q, bool kmajor, int rows, int u, int ld) {
+        if (kmajor) {
+            const int cpr = rows / 8;                 // chunks per k row
+            const int c = u * 64 + lane;
+            const int r = c / cpr;
+            const int chunk = rows >= 64 ? (c % cpr) ^ kmajor_key(r) : c % cpr;
+            voff[q] = unsigned(r) * unsigned(ld) * 2u + unsigned(chunk) * 16u;
+            kofs[q] = 0;
+        } else {
+            const int row = u * 8 + lane / 8;
+            const int chunk = (lane % 8) ^ row_key<kStep>(row);
+            voff[q] = unsigned(row) * unsigned(ld) * 2u + unsigned(chunk) * 16u;
+            kofs[q] = chunk * 8;
+        }
+    };
+#pragma unroll
+    for (int q = 0; q < PER; ++q) {
+        const int v = q * NW + wave;
+        if (of_x(q)) place(q, kXM, BM, v, a_ld);
+        else place(q, kWM, BN, v - kLoadsA, b_ld);
+    }
+    auto clamp32 = [](size_t v) { return v < 0xffffffffu ? unsigned(v) : 0xffffffffu; };
+    // Loads step k0 into stage st. Steps past the last one load nothing (an
+    // empty resource), so that every wait counts the same loads.
+    auto issue = [&](int k0, int st) {
+        const bool live = k0 < k_end;
+        const size_t ka = kXM ? size_t(k0) * a_ld : 0, kb = kWM ? size_t(k0) * b_ld : 0;
+        const auto ra = __builtin_amdgcn_make_buffer_rsrc(
+            uniform_ptr(a + ka), 0, live ? clamp32(a_bytes - ka * 2) : 0u, 0x00020000);
+        const auto rb = __builtin_amdgcn_make_buffer_rsrc(
+            uniform_ptr(b + kb), 0, live ? clamp32(b_bytes - kb * 2) : 0u, 0x00020000);
+        const int left = k_end - k0;
+#pragma unroll
+        for (int q = 0; q < PER; ++q) {
+            const int v = q * NW + wave;
+            lds_half* dst = (lds_half*)(lds + st * kStage + v * 512);
+            auto load = [&](const auto& rsrc, bool kmajor) {
+                const unsigned off = kmajor || kofs[q] < left ? voff[q] : kOutside;
+                __builtin_amdgcn_raw_ptr_buffer_load_lds(
+                    rsrc, (__attribute__((address_space(3))) void*)dst, 16, off,
+                    kmajor ? 0u : unsigned(k0) * 2u, 0, 0);
+            };
+            if (of_x(q)) load(ra, kXM);
+            else load(rb, kWM);
+        }
+    };
+
+    // ---- the epilogue's chunks: kCh consecutive columns of a row, each
+    // thread kChunks of them; their inputs load now.
+    constexpr int kCh = BM * BN >= 8 * T ? 8 : 4;
+    constexpr int kCpr = BN / kCh, kTileChunks = BM * BN / kCh;
+    constexpr int kChunks = (kTileChunks + T - 1) / T;
+    // Whole chunks only, unless n leaves a partial one (NT alone; others have
+    // n % 8 == 0).
+    const bool whole = L != Layout::kNT || n % kCh == 0;
+    const bool accumulate = ST == Store::kTn && !split && op.accumulate;
+    float aux[kF32 || ST == Store::kDGelu ? kChunks : 1][kCh];
+    float bias[kBias ? kChunks : 1][kCh];
+#pragma unroll
+    for (int i = 0; i < kChunks; ++i) {
+        const int c = i * T + tid;
+        const int row = c < kTileChunks ? m0 + c / kCpr : m, col = n0 + c % kCpr * kCh;
+        const int cols = row < m ? n - col : 0;       // valid columns from col on
+        const size_t at = y_off + size_t(row) * y_ld + col;
+        if constexpr (kBias) {
+            if (whole) {
+#pragma unroll
+                for (int e = 0; e < kCh; e += 4) {
+                    f32x4 v = {0.0f, 0.0f, 0.0f, 0.0f};
+                    if (cols > 0) v = *reinterpret_cast<const f32x4*>(op.bias + col + e);
+#pragma unroll
+                    for (int j = 0; j < 4; ++j) bias[i][e + j] = v[j];
+                }
+            } else {
+#pragma unroll
+                for (int e = 0; e < kCh; ++e) bias[i][e] = e < cols ? op.bias[col + e] : 0.0f;
+            }
+        }
+        if constexpr (kF32) {
+            const float* src = ST == Store::kTn ? static_cast<const float*>(op.y)
+                                                : static_cast<const float*>(op.aux);
+            const bool reads = ST == Store::kBiasResidual || accumulate;
+            if (whole) {
+#pragma unroll
+                for (int e = 0; e < kCh; e += 4) {
+                    f32x4 v = {0.0f, 0.0f, 0.0f, 0.0f};
+                    if (reads && cols > 0) v = *reinterpret_cast<const f32x4*>(src + at + e);
+#pragma unroll
+                    for (int j = 0; j < 4; ++j) aux[i][e + j] = v[j];
+                }
+            } else {
+#pragma unroll
+                for (int e = 0; e < kCh; ++e) aux[i][e] = reads && e < cols ? src[at + e] : 0.0f;
+            }
+        }
+        if constexpr (ST == Store::kDGelu) {
+            const _Float16* src = static_cast<const _Float16*>(op.aux) + at;
+#pragma unroll
+            for (int e = 0; e < kCh; e += 4) {
+                f16x4 v = {};
+                if (cols > 0) v = *reinterpret_cast<const f16x4*>(src + e);
+#pragma unroll
+                for (int j = 0; j < 4; ++j) aux[i][e + j] = float(v[j]);
+            }
+        }
+    }
+
+    // ---- k-loop
+    const bool computes = wave < WM * WN;
+    const int wm = wave / WN, wn = wave % WN;
+    const int fr = lane & 31, fc = lane >> 5;
+    f32x16 acc = {};
+    // Fragment of operand rows r0 .. r0 + 31, k16 sub-step kk: lane l gets row
+    // r0 + l % 32, k 8 (l / 32) .. + 8.
+    auto frag_rowmajor = [&](const _Float16* region, int r0, int kk) {
+        const int row = r0 + fr;
+        return *reinterpret_cast<const f16x8*>(region + row * kStep +
+                                               (((kk * 2 + fc) ^ row_key<kStep>(row)) * 8));
+    };
+    // Two transposing reads (inline asm: see gemm_pipe.hip). Their results are
+    // not there until wait_frags; every use comes after one, and so does every
+    // way out of the loop. A 32-row region's rows are 64 bytes: the four that
+    // 32 lanes read are consecutive, so it needs no swizzle.
+    auto frag_kmajor = [&](const _Float16* region, auto rows_c, int r0, int kk) {
+        constexpr int rows = decltype(rows_c)::value;
+        const int j = lane & 15;
+        const int col = r0 + 16 * ((lane >> 4) & 1) + 4 * (j & 3);
+        const int key = rows >= 64 ? kmajor_key(j >> 2) : 0;
+        const int chunk = ((col >> 3) ^ key) * 8 + (col & 4);
+        const int k = kk * 16 + 8 * fc + (j >> 2);
+        const unsigned a0 =
+            unsigned(reinterpret_cast<uintptr_t>((lds_half*)(region + k * rows + chunk)));
+        TrFrag f;
+        asm volatile("ds_read_b64_tr_b16 %0, %1" : "=v"(f.lo) : "v"(a0));
+        asm volatile("ds_read_b64_tr_b16 %0, %1 offset:%2" : "=v"(f.hi) : "v"(a0), "i"(4 * rows * 2));
+        return f;
+    };
+    // Waits for a step's fragments. The empty asm uses the transposing reads'
+    // registers, so that they stay theirs while the reads are in flight, also
+    // where nothing uses the values (after the last step).
+    auto wait_frags = [&](const XFrag (&x)[4], const WFrag (&w)[4]) {
+        __builtin_amdgcn_sched_barrier(0);
+        __builtin_amdgcn_s_waitcnt(0xc07f);   // lgkmcnt(0)
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int kk = 0; kk < 4; ++kk) {
+            if constexpr (kXM) asm volatile("" ::"v"(x[kk].lo), "v"(x[kk].hi));
+            if constexpr (kWM) asm volatile("" ::"v"(w[kk].lo), "v"(w[kk].hi));
+        }
+    };
+    XFrag xf[2][4];
+    WFrag wf[2][4];
+    auto read_frag = [&](int st, int kk, XFrag (&x)[4], WFrag (&w)[4]) {
+        const _Float16* s0 = lds + st * kStage;
+        if constexpr (kXM) x[kk] = frag_kmajor(s0, std::integral_constant<int, BM>{}, wm * 32, kk);
+        else x[kk] = frag_rowmajor(s0, wm * 32, kk);
+        if constexpr (kWM)
+            w[kk] = frag_kmajor(s0 + BM * kStep, std::integral_constant<int, BN>{}, wn * 32, kk);
+        else w[kk] = frag_rowmajor(s0 + BM * kStep, wn * 32, kk);
+    };
+
+    // Groups of U steps; a last group's steps past k_end add zeros.
+    const int groups = (k_end - k_begin + U * kStep - 1) / (U * kStep);
+    int k0 = k_begin;
+#pragma unroll
+    for (int j = 0; j < S; ++j, k0 += kStep) issue(k0, j);
+    wait_vmcnt<(S / U - 1) * kGroupLoads>();
+    block_sync();
+    if (computes) {
+#pragma unroll
+        for (int kk = 0; kk < 4; ++kk) read_frag(0, kk, xf[0], wf[0]);
+        wait_frags(xf[0], wf[0]);
+    }
+    int st = 0;   // the stage of the step whose fragments are in registers
+    // One step: four MFMAs with the next step's fragment reads between them (a
+    // burst of reads before the MFMAs cost a third of the step). Before a
+    // group's last step reads on, the next group has landed for every wave,
+    // and every wave holds the last step's fragments, so the group's stages
+    // take the loads of the group S / U further on; its first MFMA runs under
+    // that barrier.
+    auto step = [&](bool last, XFrag (&x)[4], WFrag (&w)[4], XFrag (&xn)[4], WFrag (&wn_)[4]) {
+        auto mfma = [&](int kk) {
+            acc = __builtin_amdgcn_mfma_f32_32x32x16_f16(as_f16x8(w[kk]), as_f16x8(x[kk]), acc, 0, 0,
+                                                         0);
+            __builtin_amdgcn_sched_barrier(0);
+        };
+        if (computes) mfma(0);
+        if (last) {
+            wait_vmcnt<(S / U - 2) * kGroupLoads>();
+            block_sync();
+#pragma unroll
+            for (int j = 0; j < U; ++j, k0 += kStep) issue(k0, st - (U - 1) + j);
+        }
+        st = st + 1 == S ? 0 : st + 1;
+        if (computes) {
+            __builtin_amdgcn_sched_barrier(0);
+            read_frag(st, 0, xn, wn_);
+            read_frag(st, 1, xn, wn_);
+            __builtin_amdgcn_sched_barrier(0);
+            mfma(1);
+            read_frag(st, 2, xn, wn_);
+            __builtin_amdgcn_sched_barrier(0);
+            mfma(2);
+            read_frag(st, 3, xn, wn_);
+            __builtin_amdgcn_sched_barrier(0);
+            mfma(3);
+            wait_frags(xn, wn_);
+        }
+    };
+    if constexpr (U == 1) {
+        for (int g = 0; g < groups; g += 2) {
+            step(true, xf[0], wf[0], xf[1], wf[1]);
+            if (g + 1 < groups) step(true, xf[1], wf[1], xf[0], wf[0]);
+        }
+    } else {
+        static_assert(U % 2 == 0, "fragment buffers alternate within a group");
+        for (int g = 0; g < groups; ++g) {
+#pragma unroll
+            for (int j = 0; j < U; j += 2) {
+                step(false, xf[0], wf[0], xf[1], wf[1]);
+                step(j + 2 == U, xf[1], wf[1], xf[0], wf[0]);
+            }
+        }
+    }
+
+    // ---- epilogue: the sums through LDS (the stages, once every load into
+    // them has landed), then whole chunks.
+    wait_vmcnt<0>();
+    block_sync();
+    float* const sums = reinterpret_cast<float*>(lds);
+    if (computes) {
+#pragma unroll
+        for (int g4 = 0; g4 < 4; ++g4) {
+            const f32x4 v = {acc[g4 * 4 + 0], acc[g4 * 4 + 1], acc[g4 * 4 + 2], acc[g4 * 4 + 3]};
+            *reinterpret_cast<f32x4*>(sums + (wm * 32 + fr) * kLd + wn * 32 + g4 * 8 + fc * 4) = v;
+        }
+    }
+    block_sync();
+#pragma unroll
+    for (int i = 0; i < kChunks; ++i) {
+        const int c = i * T + tid;
+        const int r = c / kCpr, cc = c % kCpr * kCh;
+        const int row = m0 + r, col = n0 + cc;
+        if (c >= kTileChunks || row >= m || col >= n) continue;
+        float v[kCh];
+#pragma unroll
+        for (int e = 0; e < kCh; e += 4) {
+            const f32x4 s4 = *reinterpret_cast<const f32x4*>(sums + r * kLd + cc + e);
+#pragma unroll
+            for (int j = 0; j < 4; ++j) v[e + j] = s4[j];
+        }
+        const size_t at = y_off + size_t(row) * y_ld + col;
+        const int cols = n - col;
+        typedef _Float16 hch __attribute__((ext_vector_type(kCh)));
+        auto store_half = [&](void* out, const hch& h) {
+            _Float16* p = static_cast<_Float16*>(out) + at;
+            if (whole) {
+                *reinterpret_cast<hch*>(p) = h;
+            } else {
+#pragma unroll
+                for (int e = 0; e < kCh; ++e)
+                    if (e < cols) p[e] = h[e];
+            }
+        };
+        if constexpr (kF32) {
+            if constexpr (ST == Store::kBiasResidual) {
+#pragma unroll
+                for (int e = 0; e < kCh; ++e) v[e] = aux[i][e] + (v[e] + bias[i][e]);
+            } else if (accumulate) {
+#pragma unroll
+                for (int e = 0; e < kCh; ++e) v[e] = aux[i][e] + v[e];
+            }
+            float* p = (split ? op.partials : static_cast<float*>(op.y)) + at;
+            if (whole) {
+#pragma unroll
+                for (int e = 0; e < kCh; e += 4)
+                    *reinterpret_cast<f32x4*>(p + e) = f32x4{v[e], v[e + 1], v[e + 2], v[e + 3]};
+            } else {
+#pragma unroll
+                for (int e = 0; e < kCh; ++e)
+                    if (e < cols) p[e] = v[e];
+            }
+        } else {
+            hch h;
+            if constexpr (kBias) {
+#pragma unroll
+                for (int e = 0; e < kCh; ++e) v[e] = settled(v[e] + bias[i][e]);
+            }
+            if constexpr (ST == Store::kScale) {
+#pragma unroll
+                for (int e = 0; e < kCh; ++e) v[e] = settled(v[e] * op.scale);
+            }
+            if constexpr (ST == Store::kDGelu) {
+#pragma unroll
+                for (int e = 0; e < kCh; ++e) v[e] = settled(v[e] * gelu_grad(aux[i][e]));
+            }
+#pragma unroll
+            for (int e = 0; e < kCh; ++e) h[e] = _Float16(v[e]);
+            store_half(ST == Store::kBiasGelu ? op.aux : op.y, h);
+            if constexpr (ST == Store::kBiasGelu) {
+#pragma unroll
+                for (int e = 0; e < kCh; ++e) h[e] = _Float16(settled(gelu(v[e])));
+                store_half(op.y, h);
+            }
+        }
+    }
+#endif
+}
+
+// A configuration and its cost, measured on one MI355X (us; operands rotated
+// past the caches): `alone` is a k-step of a tile that has its CU to itself,
+// `shared` a k-step's share of the CU when there are more tiles than CUs,
+// `fixed` a tile's prologue and epilogue. Each per layout NT, NN, TN.
+struct SmallConfig {
+    int bm, bn, waves, stages, unit;
+    double alone[3], shared[3], fixed;
+};
+constexpr SmallConfig kSmallConfigs[] = {
+    // Least to stream per CU: the smallest products.
+    {32, 32, 4, 8, 2, {0.135, 0.19, 0.20}, {0.145, 0.20, 0.21}, 0.7},
+    // The same for up to twice the tiles.
+    {32, 64, 4, 6, 2, {0.16, 0.20, 0.24}, {0.19, 0.20, 0.26}, 0.8},
+    // Eight waves load for one tile a CU: long k-ranges.
+    {64, 64, 8, 8, 2, {0.19, 0.235, 0.28}, {0.30, 0.33, 0.37}, 1.3},
+    // Two tiles a CU.
+    {64, 64, 4, 4, 1, {0.25, 0.26, 0.28}, {0.25, 0.25, 0.27}, 1.0},
+    // The fewest operand bytes per output: many tiles.
+    {128, 64, 8, 3, 1, {0.30, 0.34, 0.40}, {0.44, 0.44, 0.44}, 1.3},
+};
+
+int layout_index(GemmLayout l) { return l == GemmLayout::kNT ? 0 : (l == GemmLayout::kNN ? 1 : 2); }
+
+// Estimated us (past a launch's own) of `tiles` tiles of `steps` k-steps.
+double small_cost(const SmallConfig& c, GemmLayout l, double tiles, double steps, int cus) {
+    const int i = layout_index(l);
+    const double load = tiles / cus;
+    if (load <= 1.0) return c.fixed + steps * c.alone[i];
+    const double shares = load <= 2.0 ? 2.0 : load;
+    return shares * (c.fixed + steps * c.shared[i]);
+}
+
+double small_tiles(const SmallConfig& c, size_t slices, size_t m, size_t n) {
+    return double((m + c.bm - 1) / c.bm) * double((n + c.bn - 1) / c.bn) * double(slices);
+}
+
+// The "gemm_small" override: "0" turns these kernels off,
+// "bm,bn,waves,stages,unit" takes that configuration for every product.
+bool small_forced(SmallConfig* out, bool* disabled) {
+    *disabled = false;
+    const char* e = tuning(Tune::kGemmSmall);
+    if (e == nullptr) return false;
+    if (e[0] == '0' && e[1] == '\0') {
+        *disabled = true;
+        return false;
+    }
+    SmallConfig c{};
+    if (std::sscanf(e, "%d,%d,%d,%d,%d", &c.bm, &c.bn, &c.waves, &c.stages, &c.unit) != 5)
+        return false;
+    for (const SmallConfig& k : kSmallConfigs) {
+        if (k.bm == c.bm && k.bn == c.bn && k.waves == c.waves && k.stages == c.stages &&
+            k.unit == c.unit) {
+            *out = k;
+            return true;
+        }
+    }
+    return false;
+}
+
+template <Layout L, Store ST, bool HV>
+hipError_t launch(const SmallPlan& c, const Operands& op, size_t slices, hipStream_t stream) {
+    TileArgs ta{};
+    ta.tiles_m = (op.m + c.bm - 1) / c.bm;
+    ta.tiles_n = (op.n + c.bn - 1) / c.bn;
+    const size_t per = size_t(ta.tiles_m) * size_t(ta.tiles_n);
+    if (per * slices > 0x7fffffffu) return hipErrorInvalidValue;
+    ta.tiles_per_slice = int(per);
+    ta.slices = int(slices);
+    ta.group_m = 8;
+    ta.split_len = c.split_len;
+    const dim3 grid(unsigned(per * slices));
+#define FLINT_SMALL_CASE(BM_, BN_, NW_, S_, U_)                                                    \
+    if (c.bm == BM_ && c.bn == BN_ && c.waves == NW_ && c.stages == S_ && c.unit == U_) {          \
+        hipLaunchKernelGGL((gemm_small<BM_ / 32, BN_ / 32, NW_, S_, U_, L, ST, HV>), grid,         \
+                           dim3(NW_ * 64), 0, stream, op, ta);                                     \
+        return hipGetLastError();                                                                  \
+    }
+    FLINT_SMALL_CASE(32, 32, 4, 8, 2)
+    FLINT_SMALL_CASE(32, 64, 4, 6, 2)
+    FLINT_SMALL_CASE(64, 64, 8, 8, 2)
+    FLINT_SMALL_CASE(64, 64, 4, 4, 1)
+    FLINT_SMALL_CASE(128, 64, 8, 3, 1)
+#undef FLINT_SMALL_CASE
+    return hipErrorInvalidValue;
+}
+
+}  // namespace
+
+// Whether these kernels take a product, and with which tile and TN split:
+// where the cheapest configuration costs less than gemm_pipe.hip's choice, by
+// the estimates of both (gemm_pipe_estimate; infinite where the pipeline does
+// not take the shape). Either side gives the same sums, so the line only has
+// to be about right.
+bool gemm_small_plan(GemmLayout l, Epilogue e, size_t slices, size_t m, size_t n, size_t k,
+                     int max_splits, SmallPlan* plan) {
+    SmallConfig forced;
+    bool disabled = false;
+    const bool force = small_forced(&forced, &disabled);
+    if (disabled || m == 0 || n == 0 || k == 0) return false;
+    // A forced pipeline tile means the pipeline.
+    if (!force && tuning(Tune::kGemmPipe) != nullptr) return false;
+    int cus = 256;
+    if (device_cus(&cus) != hipSuccess) return false;
+    double best = force ? kNoEstimate : gemm_pipe_estimate(l, e, slices, m, n, k, max_splits);
+    // Ragged products the pipeline does not take would run gemm.hip's kernels:
+    // slower up to about 60 rounds of 128 x 64 tiles (NT 2500 x 50257 x 768 465
+    // against 446 us here; 6753 x 800 x 200 14.9 against 11.2), faster at 196
+    // (8192 x 50257 x 768 1486 against 1592).
+    if (best == kNoEstimate && !force && small_tiles(kSmallConfigs[4], slices, m, n) > 96.0 * cus)
+        return false;
+    bool taken = false;
+    for (const SmallConfig& c : kSmallConfigs) {
+        if (force && (c.bm != forced.bm || c.bn != forced.bn || c.waves != forced.waves)) continue;
+        const double tiles = small_tiles(c, slices, m, n);
+        if (tiles > double(0x7fffffff)) continue;
+        for (int sp = 1; sp <= max_splits; ++sp) {
+            const size_t len = ((k + sp - 1) / sp + kStep - 1) / kStep * kStep;
+            if (size_t(sp - 1) * len >= k || tiles * sp > double(0x7fffffff)) break;
+            double cost = small_cost(c, l, tiles * sp, double(len / kStep), cus);
+            if (sp > 1) cost += kSplitSumUs + double(sp + 2) * double(m) * double(n) * 4.0 / 5e6;
+            if (cost < best) {
+                best = cost;
+                taken = true;
+                *plan = {c.bm, c.bn, c.waves, c.stages, c.unit, sp, int(len)};
+            }
+        }
+    }
+    return taken;
+}
+
+hipError_t launch_gemm_small(const SmallPlan& c, GemmLayout l, Epilogue e, void* y, const void* x,
+                             const void* w, const void* bias, void* aux, float scale,
+                             size_t slices, size_t m, size_t n, size_t k, bool accumulate,
+                             void* partials, hipStream_t stream, bool causal, const HeadView* wv,
+                             const HeadView* yv) {
+    Operands op{};
+    op.y = y;
+    op.x = static_cast<const _Float16*>(x);
+    op.w = static_cast<const _Float16*>(w);
+    op.bias = static_cast<const float*>(bias);
+    op.aux = aux;
+    op.partials = static_cast<float*>(partials);
+    op.scale = scale;
+    op.accumulate = accumulate ? 1 : 0;
+    op.m = int(m);
+    op.n = int(n);
+    op.k = int(k);
+    op.causal = causal ? 1 : 0;
+    const bool hv = wv != nullptr && yv != nullptr;
+    if (hv) {
+        op.wv = *wv;
+        op.yv = *yv;
+    }
+    if (l == GemmLayout::kNT) {
+        switch (e) {
+        case Epilogue::kNone: return launch<Layout::kNT, Store::kNone, false>(c, op, slices, stream);
+        case Epilogue::kBias: return launch<Layout::kNT, Store::kBias, false>(c, op, slices, stream);
+        case Epilogue::kBiasGelu:
+            return launch<Layout::kNT, Store::kBiasGelu, false>(c, op, slices, stream);
+        case Epilogue::kBiasResidual:
+            return launch<Layout::kNT, Store::kBiasResidual, false>(c, op, slices, stream);
+        case Epilogue::kScale: return launch<Layout::kNT, Store::kScale, false>(c, op, slices, stream);
+        default: return hipErrorInvalidValue;
+        }
+    }
+    if (l == GemmLayout::kNN) {
+        if (e == Epilogue::kDGelu) return launch<Layout::kNN, Store::kDGelu, false>(c, op, slices, stream);
+        if (e != Epilogue::kNone) return hipErrorInvalidValue;
+        return hv ? launch<Layout::kNN, Store::kNone, true>(c, op, slices, stream)
+                  : launch<Layout::kNN, Store::kNone, false>(c, op, slices, stream);
+    }
+    if (e == kTnFloat) return launch<Layout::kTN, Store::kTn, false>(c, op, size_t(c.splits), stream);
+    if (e != Epilogue::kNone) return hipErrorInvalidValue;
+    return hv ? launch<Layout::kTN, Store::kTnHalf, true>(c, op, slices, stream)
+              : launch<Layout::kTN, Store::kTnHalf, false>(c, op, slices, stream);
+}
+
+}  // namespace flint

@@ -47,6 +47,27 @@ hipError_t launch_gemm_pipe(GemmLayout l, Epilogue e, void* y, const void* x, co
                             size_t n, size_t k, bool accumulate, void* partials, int split_len,
                             hipStream_t stream, bool causal = false,
                             const HeadView* wv = nullptr, const HeadView* yv = nullptr);
+// The pipeline's estimated time for a product, us past a launch's own, with
+// the tile (and TN split, up to max_splits) it would choose; infinite where it
+// does not take the shape.
+double gemm_pipe_estimate(GemmLayout l, Epilogue e, size_t slices, size_t m, size_t n, size_t k,
+                          int max_splits);
+// GEMMs of few tiles (gemm_small.hip), every layout, epilogue and size: the
+// launchers below run there where gemm_small_plan says so. max_splits: TN's
+// FP32 output may split k up to that often (the count is plan->splits, the
+// partials, when there are several, in `partials`); 1 otherwise. The other
+// arguments are launch_gemm_pipe's; views come in pairs.
+struct SmallPlan {
+    int bm, bn, waves, stages, unit;
+    int splits, split_len;
+};
+bool gemm_small_plan(GemmLayout l, Epilogue e, size_t slices, size_t m, size_t n, size_t k,
+                     int max_splits, SmallPlan* plan);
+hipError_t launch_gemm_small(const SmallPlan& plan, GemmLayout l, Epilogue e, void* y, const void* x,
+                             const void* w, const void* bias, void* aux, float scale,
+                             size_t slices, size_t m, size_t n, size_t k, bool accumulate,
+                             void* partials, hipStream_t stream, bool causal = false,
+                             const HeadView* wv = nullptr, const HeadView* yv = nullptr);
 hipError_t launch_gemm_nn(void* y, const void* x, const void* w, const void* aux, Epilogue e,
                           size_t m, size_t n, size_t k, hipStream_t stream);
 // Number of k splits TN uses for m x n x k on this device (1 = none).

@@ -9,6 +9,7 @@
  *
  * Names and values:
  *   "gemm_pipe"     "0" (no pipeline kernel) or "bm,bn,stages[,bk[,waves[,loaders]]]"
+ *   "gemm_small"    "0" (no few-tile kernel) or "bm,bn,waves,stages,unit"
  *   "gemm_config"   "bm,bn,bk,stages,waves_m[,waves]" (the non-pipeline kernel)
  *   "gemm_group_m", "gemm_slots"   positive integers (the non-pipeline kernel)
  *   "attn_causal", "fused_grads", "fused_sums", "ln_defer", "ln_fused",
