@@ -144,13 +144,27 @@ def pointer(value):
 
 
 def stream_handle(stream):
+    if stream is None:
+        return _current_stream()
     if isinstance(stream, int):
         return stream
+    return stream.cuda_stream
+
+
+def _current_stream():
+    """torch's current stream on the calling thread, as a handle. Asked of torch
+    directly: torch.cuda.current_stream() builds a Stream object, 3.0 us of a
+    call's 7.4 (this way 0.2 us, a call 4.7). It also initialises torch's HIP
+    state, so the first call here goes through it."""
+    global _current_stream
     import torch
 
-    if stream is None:
-        return torch.cuda.current_stream().cuda_stream
-    return stream.cuda_stream
+    handle = torch.cuda.current_stream().cuda_stream
+    device = getattr(torch._C, "_cuda_getDevice", None)
+    raw = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+    if device is not None and raw is not None:
+        _current_stream = lambda: raw(device())  # noqa: E731
+    return handle
 
 
 def library_path():
