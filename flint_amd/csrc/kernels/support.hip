@@ -5,6 +5,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <type_traits>
 #include <cstdint>
 #include <cstdlib>
 
@@ -540,56 +541,110 @@ column_sums_one_chunk(float* __restrict__ out, const float* __restrict__ dy, int
 // ------------------------------------------------ token rows without a sort
 
 constexpr int kScanRows = 8192;   // tokens embedding_scan_runs holds in LDS
-constexpr int kScanWaves = 4;     // positions (one a wave) per workgroup
+constexpr int kScanWaves = 8;     // positions (one a wave) per workgroup
 constexpr int kScanThreads = kScanWaves * 64;
-constexpr int kScanBatch = 4;     // rows of a run whose loads go out together
+constexpr int kScanBlock = 512;   // positions a wave tests at a time, 8 a lane
+constexpr int kScanBlocks = kScanRows / kScanBlock;
+constexpr int kScanBatch = 4;     // rows of a short run whose loads go out together
+constexpr int kScanShort = 16;    // the longest run one wave sums by itself
+constexpr int kScanLongBatch = 16;   // rows of a long run in flight, twice over
 
-// The positions of one 512-position block of the scan that hold a token:
-// bit l of m[k] says whether lane l's position 8 l + k does. next() returns
-// them in ascending order (base + 8 l + k), then -1. Every member holds the
-// same value on all lanes.
+typedef uint16_t u16x8 __attribute__((ext_vector_type(8)));
+// Lane l's word of the block at base.
+__device__ __forceinline__ u16x8 scan_word(const uint16_t* tok, int base, int lane) {
+    return *reinterpret_cast<const u16x8*>(tok + base + 8 * lane);
+}
+
+// The positions of one block of the scan that hold a token, as ballots: bit l
+// of m[k] says whether position base + 8 l + k does. Lane order is position
+// order.
 struct BlockMatches {
     uint64_t m[8];
-    uint64_t lanes;   // lanes with a position not yet returned, but `at`
-    unsigned cur;     // positions k of lane `at` not yet returned
-    int at;
-    int base;
-    __device__ int next() {
-        if (cur == 0) {
-            if (lanes == 0) return -1;
-            at = __builtin_ctzll(lanes);
-            lanes &= lanes - 1;
+    // t: the lane's word, positions base + 8 lane .. + 7 (inside tok, as base +
+    // 512 <= kScanRows); positions at or past rows, in the last block, are
+    // masked off.
+    __device__ __forceinline__ void test(const u16x8& t, int base, int rows, uint16_t v, int lane) {
 #pragma unroll
-            for (int k = 0; k < 8; ++k) cur |= unsigned((m[k] >> at) & 1) << k;
+        for (int k = 0; k < 8; ++k) m[k] = __builtin_amdgcn_ballot_w64(t[k] == v);
+        if (base + kScanBlock > rows) {
+            const int left = rows - base - 8 * lane;
+#pragma unroll
+            for (int k = 0; k < 8; ++k) m[k] &= __builtin_amdgcn_ballot_w64(k < left);
         }
-        const int k = __builtin_ctz(cur);
-        cur &= cur - 1;
-        return base + 8 * at + k;
+    }
+    __device__ __forceinline__ uint64_t any() const {
+        return (m[0] | m[1] | m[2] | m[3]) | (m[4] | m[5] | m[6] | m[7]);
+    }
+    __device__ __forceinline__ int count() const {
+        int n = 0;
+#pragma unroll
+        for (int k = 0; k < 8; ++k) n += __builtin_popcountll(m[k]);
+        return n;
+    }
+    // The first of them (any() != 0).
+    __device__ __forceinline__ int first(int base) const {
+        const int l = __builtin_ctzll(any());
+        unsigned at = 0;   // bit k: position k of lane l (no index into m: it stays in registers)
+#pragma unroll
+        for (int k = 0; k < 8; ++k) at |= unsigned((m[k] >> l) & 1) << k;
+        return base + 8 * l + __builtin_ctz(at);
+    }
+    // Writes them in ascending order to list[at], list[at + 1], ...: a lane's
+    // rank is the matches of the lanes below it. Entries from `cap` on are
+    // left out.
+    __device__ __forceinline__ void append(uint16_t* list, int at, int cap, int base, int lane) const {
+        const uint64_t below = (uint64_t{1} << lane) - 1;
+        int rank = at;
+#pragma unroll
+        for (int k = 0; k < 8; ++k) rank += __builtin_popcountll(m[k] & below);
+#pragma unroll
+        for (int k = 0; k < 8; ++k) {
+            if ((m[k] >> lane) & 1) {
+                if (rank < cap) list[rank] = uint16_t(base + 8 * lane + k);
+                ++rank;
+            }
+        }
     }
 };
 
+__device__ __forceinline__ float run_value(float old, const Comp& s) {
+    return add_rn(old, __builtin_isfinite(s.sum) ? add_rn(s.sum, s.error) : s.sum);
+}
+
 // dwte += the token rows of dx without sorting them (up to kScanRows rows,
-// widths up to 256 G). The tokens sit in LDS, and wave w of workgroup b takes
-// position i = kScanWaves b + w. The wave scans the tokens in ascending
-// blocks of 512, lane l reading positions 8 l .. 8 l + 7 of a block as one
-// 16-byte word, so that lane order is position order. If the first block
-// holding the wave's token holds it before i, an earlier position's wave owns
-// the token and this one leaves. Otherwise i is the token's first position:
-// the wave adds the dx rows of i and of every later position with the same
-// token, in ascending order, kScanBatch rows' loads in flight at a time. That
-// is the run a stable sort puts together, summed as embedding_runs sums it
-// (compensated, in the same order), so the bits are the sorted path's. Lane l
-// holds columns 256 g + 4 l (g < G). Workgroups from run_blocks on take
-// column quads of the position gradient (column_sums_quad, as in
-// sort_tokens_and_positions).
+// widths up to 256 G). Each position is one wave's: the tokens sit in LDS, and
+// the wave scans them in ascending blocks of 512, lane l testing positions
+// 8 l .. 8 l + 7 of a block, which ballots turn into the positions that hold
+// its token. If one is below its own, that position's wave owns the token and
+// this one is done. Otherwise the wave owns the run: its position and every
+// later one with the token, in ascending order -- the run that a stable sort
+// puts together, summed as embedding_runs sums it (compensated, in the same
+// order), so the bits are the sorted path's.
+//  * A short run (up to 16 rows) is the owner's alone: lane l holds columns
+//    256 g + 4 l (g < G), kScanBatch rows' loads in flight.
+//  * A longer one is a serial chain whose arithmetic one wave would take 340
+//    cycles a row for (G = 3), so it is the whole workgroup's: the waves list
+//    its rows together (each scans two blocks), and then each thread sums one
+//    or two columns, 16 rows' loads in flight while 16 are added.
+// Text has few frequent words and they all start near the front: positions
+// are dealt to workgroups a grid apart, so that their runs spread over the
+// GPU. At 8 x 1024 x 768 (one MI355X, position sums included): text-like
+// tokens (257 rows of the most frequent) 114.5 -> 27.1 us against one wave a
+// run at every length,
+// uniform ones 23.0 -> 24.1, Zipf s = 1.1 (a run of 1,113) 441 -> 77.
+// Workgroups from run_blocks on take column quads of the position gradient
+// (column_sums_quad, as in sort_tokens_and_positions).
 template <int G>
-__global__ void __launch_bounds__(kScanThreads)
+__global__ void __launch_bounds__(kScanThreads) __attribute__((amdgpu_waves_per_eu(4, 4)))
 embedding_scan_runs(float* __restrict__ dwte, const float* __restrict__ dx,
                     const uint16_t* __restrict__ tokens, int rows, size_t width,
                     unsigned run_blocks, float* __restrict__ dwpe, int sequences, size_t cols,
                     int accumulate_wpe) {
-    typedef uint16_t u16x8 __attribute__((ext_vector_type(8)));
     __shared__ __attribute__((aligned(16))) uint16_t tok[kScanRows];
+    __shared__ uint16_t shorts[kScanWaves][kScanShort];   // a short run's rows
+    __shared__ uint16_t longs[kScanRows];                 // a long run's
+    __shared__ int runs[kScanWaves];                      // a wave's run if it is long, else 0
+    __shared__ int counts[kScanBlocks];
     if (blockIdx.x >= run_blocks) {
         column_sums_quad(dwpe, dx, sequences, cols, accumulate_wpe,
                          size_t(blockIdx.x - run_blocks) * kScanThreads + threadIdx.x);
@@ -602,83 +657,164 @@ embedding_scan_runs(float* __restrict__ dwte, const float* __restrict__ dx,
     for (int p = words * 8 + int(threadIdx.x); p < rows; p += kScanThreads) tok[p] = tokens[p];
     __syncthreads();
     const int lane = int(threadIdx.x & 63);
-    const size_t col0 = size_t(lane) * 4;
-    const int i = int(blockIdx.x) * kScanWaves + int(threadIdx.x >> 6);
-    if (i >= rows) return;
-    const uint16_t v = tok[i];
-    Comp s[G][4];
-    f4 old[G];
-    bool owner = false;
-    // Each block's word is read while the one before is tested. base + 8 lane
-    // + 7 < base + 512 <= kScanRows: the word stays inside tok; positions at
-    // or past rows are masked off.
-    u16x8 next = *reinterpret_cast<const u16x8*>(tok + 8 * lane);
-    for (int base = 0; base < rows; base += 512) {
-        const u16x8 t = next;
-        if (base + 512 < rows) next = *reinterpret_cast<const u16x8*>(tok + base + 512 + 8 * lane);
-        const int left = rows - base - 8 * lane;
-        BlockMatches bm;
-        bm.lanes = 0;
-        bm.cur = 0;
-        bm.at = 0;
-        bm.base = base;
-#pragma unroll
-        for (int k = 0; k < 8; ++k) bm.m[k] = __builtin_amdgcn_ballot_w64(t[k] == v);
-        if (base + 512 > rows) {   // the last block: no match at or past rows
-#pragma unroll
-            for (int k = 0; k < 8; ++k) bm.m[k] &= __builtin_amdgcn_ballot_w64(k < left);
+    const int wave = __builtin_amdgcn_readfirstlane(int(threadIdx.x >> 6));
+    const int i = wave * int(run_blocks) + int(blockIdx.x);
+    int n = 0;   // the rows of this wave's run, 0 where it owns none
+    if (i < rows) {
+        const uint16_t v = tok[i];
+        // Each block's word is read while the one before is tested.
+        u16x8 next = scan_word(tok, 0, lane);
+        for (int base = 0; base < rows; base += kScanBlock) {
+            const u16x8 t = next;
+            if (base + kScanBlock < rows) next = scan_word(tok, base + kScanBlock, lane);
+            BlockMatches bm;
+            bm.test(t, base, rows, v, lane);
+            if (bm.any() == 0) continue;
+            if (n == 0 && bm.first(base) < i) break;   // an earlier position's run
+            if (n < kScanShort) bm.append(shorts[wave], n, kScanShort, base, lane);
+            n += bm.count();
         }
+    }
+    if (lane == 0) runs[wave] = n > kScanShort ? n : 0;
+    if (n > 0 && n <= kScanShort) {
+        // Other lanes wrote the list.
+        __builtin_amdgcn_wave_barrier();
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        float* const out = dwte + size_t(tok[i]) * width;
+        const size_t col0 = size_t(lane) * 4;
+        Comp s[G][4];
+        f4 old[G];
 #pragma unroll
-        for (int k = 0; k < 8; ++k) bm.lanes |= bm.m[k];
-        if (bm.lanes == 0) continue;
-        if (!owner) {
-            BlockMatches first = bm;
-            if (first.next() < i) return;   // an earlier position holds the token
-            owner = true;
-            // The row the sums add into, loaded beside the first dx rows.
-#pragma unroll
-            for (int g = 0; g < G; ++g) {
-                const size_t col = col0 + size_t(g) * 256;
-                old[g] = col < width ? *reinterpret_cast<const f4*>(dwte + size_t(v) * width + col)
-                                     : f4{0.0f, 0.0f, 0.0f, 0.0f};
-            }
+        for (int g = 0; g < G; ++g) {
+            const size_t col = col0 + size_t(g) * 256;
+            old[g] = col < width ? *reinterpret_cast<const f4*>(out + col) : f4{0.0f, 0.0f, 0.0f, 0.0f};
         }
-        for (;;) {
-            int j[kScanBatch];
-#pragma unroll
-            for (int u = 0; u < kScanBatch; ++u) j[u] = bm.next();
+        for (int k = 0; k < n; k += kScanBatch) {
             f4 d[kScanBatch][G];
 #pragma unroll
-            for (int u = 0; u < kScanBatch; ++u)
+            for (int u = 0; u < kScanBatch; ++u) {
+                const bool live = k + u < n;
+                const size_t row = live ? size_t(__builtin_amdgcn_readfirstlane(int(shorts[wave][k + u]))) : 0;
 #pragma unroll
                 for (int g = 0; g < G; ++g) {
                     const size_t col = col0 + size_t(g) * 256;
-                    d[u][g] = j[u] >= 0 && col < width
-                                  ? *reinterpret_cast<const f4*>(dx + size_t(j[u]) * width + col)
+                    d[u][g] = live && col < width
+                                  ? *reinterpret_cast<const f4*>(dx + row * width + col)
                                   : f4{0.0f, 0.0f, 0.0f, 0.0f};
                 }
+            }
 #pragma unroll
             for (int u = 0; u < kScanBatch; ++u) {
-                if (j[u] < 0) break;
+                if (k + u >= n) break;
 #pragma unroll
                 for (int g = 0; g < G; ++g)
 #pragma unroll
                     for (int c = 0; c < 4; ++c) comp_add(s[g][c], d[u][g][c]);
             }
-            if (j[kScanBatch - 1] < 0) break;
+        }
+#pragma unroll
+        for (int g = 0; g < G; ++g) {
+            const size_t col = col0 + size_t(g) * 256;
+            if (col >= width) continue;
+            f4 r;
+#pragma unroll
+            for (int c = 0; c < 4; ++c) r[c] = run_value(old[g][c], s[g][c]);
+            *reinterpret_cast<f4*>(out + col) = r;
         }
     }
+    __syncthreads();
+    for (int owner = 0; owner < kScanWaves; ++owner) {
+        const int total = runs[owner];
+        if (total == 0) continue;   // the same for every thread
+        const uint16_t v = tok[owner * int(run_blocks) + int(blockIdx.x)];
+        // List the run's rows: the blocks' counts, then each block's rows
+        // after those of the blocks before it.
+        static_assert(kScanBlocks % kScanWaves == 0, "whole blocks per wave");
+        BlockMatches bm[kScanBlocks / kScanWaves];
 #pragma unroll
-    for (int g = 0; g < G; ++g) {
-        const size_t col = col0 + size_t(g) * 256;
-        if (col >= width) continue;
-        f4 r;
+        for (int q = 0; q < kScanBlocks / kScanWaves; ++q) {
+            const int block = q * kScanWaves + wave;
+            bm[q].test(scan_word(tok, block * kScanBlock, lane), block * kScanBlock, rows, v, lane);
+            if (lane == 0) counts[block] = bm[q].count();
+        }
+        __syncthreads();
 #pragma unroll
-        for (int c = 0; c < 4; ++c)
-            r[c] = add_rn(old[g][c], __builtin_isfinite(s[g][c].sum)
-                                         ? add_rn(s[g][c].sum, s[g][c].error)
-                                         : s[g][c].sum);
-        *reinterpret_cast<f4*>(dwte + size_t(v) * width + col) = r;
+        for (int q = 0; q < kScanBlocks / kScanWaves; ++q) {
+            const int block = q * kScanWaves + wave;
+            if (bm[q].any() == 0) continue;
+            int at = 0;
+            for (int b = 0; b < block; ++b) at += counts[b];
+            bm[q].append(longs, at, kScanRows, block * kScanBlock, lane);
+        }
+        __syncthreads();
+        // Thread t has column t and, in the waves that width leaves one for,
+        // column t + kScanThreads (waves w and w + 4 share a SIMD: at width
+        // 768 each SIMD adds 3 columns a lane). A column past the row's end
+        // loads the last one and is never stored: no branch around the loads,
+        // so that they stay in flight while the batch before is added.
+        auto sum_run = [&](auto columns) {
+            constexpr int kCols = decltype(columns)::value;
+            float* const out = dwte + size_t(v) * width;
+            unsigned at[kCols];   // bytes into a row
+            Comp s[kCols];
+            float old[kCols];
+#pragma unroll
+            for (int c = 0; c < kCols; ++c) {
+                at[c] = min(unsigned(c) * kScanThreads + threadIdx.x, unsigned(width) - 1) * 4u;
+                old[c] = *reinterpret_cast<const float*>(reinterpret_cast<const char*>(out) + at[c]);
+            }
+            // Lane l holds entry l of the list's current 64; past the run's end
+            // its last row again, loaded but not added.
+            int list = 0;
+            auto load = [&](int k, float (&to)[kScanLongBatch][kCols]) {
+                if ((k & 63) == 0) list = longs[min(k + lane, total - 1)];
+#pragma unroll
+                for (int u = 0; u < kScanLongBatch; ++u) {
+                    const unsigned row = unsigned(__builtin_amdgcn_readlane(list, (k & 63) + u));
+                    const char* p = reinterpret_cast<const char*>(dx) + uint64_t(row) * (unsigned(width) * 4u);
+#pragma unroll
+                    for (int c = 0; c < kCols; ++c) to[u][c] = *reinterpret_cast<const float*>(p + at[c]);
+                }
+            };
+            auto add = [&](const float (&from)[kScanLongBatch][kCols]) {
+#pragma unroll
+                for (int u = 0; u < kScanLongBatch; ++u)
+#pragma unroll
+                    for (int c = 0; c < kCols; ++c) comp_add(s[c], from[u][c]);
+            };
+            auto add_first = [&](int count, const float (&from)[kScanLongBatch][kCols]) {
+#pragma unroll
+                for (int u = 0; u < kScanLongBatch; ++u) {
+                    if (u < count) {
+#pragma unroll
+                        for (int c = 0; c < kCols; ++c) comp_add(s[c], from[u][c]);
+                    }
+                }
+            };
+            float d[2][kScanLongBatch][kCols];
+            int k = 0;
+            load(0, d[0]);
+            for (; k + 2 * kScanLongBatch <= total; k += 2 * kScanLongBatch) {
+                load(k + kScanLongBatch, d[1]);
+                add(d[0]);
+                load(k + 2 * kScanLongBatch, d[0]);
+                add(d[1]);
+            }
+            if (k + kScanLongBatch <= total) {
+                load(k + kScanLongBatch, d[1]);
+                add(d[0]);
+                add_first(total - k - kScanLongBatch, d[1]);
+            } else {
+                add_first(total - k, d[0]);
+            }
+#pragma unroll
+            for (int c = 0; c < kCols; ++c)
+                if (size_t(c) * kScanThreads + threadIdx.x < width)
+                    *reinterpret_cast<float*>(reinterpret_cast<char*>(out) + at[c]) = run_value(old[c], s[c]);
+        };
+        if (G > 2 && size_t(kScanThreads) + wave * 64 < width) sum_run(std::integral_constant<int, 2>{});
+        else sum_run(std::integral_constant<int, 1>{});
+        __syncthreads();   // the next run lists its rows in the same place
     }
 }
 
