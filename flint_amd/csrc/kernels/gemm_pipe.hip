@@ -173,8 +173,12 @@ __device__ inline void map_tile_causal(const TileArgs& t, unsigned id, int bm, i
 // HV (batched NN / TN only): w and y are heads views (op.wv, op.yv), rows
 // op.wv.ld / op.yv.ld apart. A template flag, so that the other instances
 // keep their scalar registers: the runtime strides alone spilled SGPRs.
+// KT (NT and NN): k is not a whole number of k-steps; the last step's chunks
+// past k read zeros (one select per load, so only these instances carry it).
+// TN needs no flag: its operands are k-major, and rows past k lie past their
+// resources' ends.
 template <int BM, int BN, int S, int BK, Layout L, Store ST, int NW, bool LD = false,
-          bool HV = false>
+          bool HV = false, bool KT = false>
 __global__ void __launch_bounds__((NW + (LD ? 4 : 0)) * 64)
 __attribute__((amdgpu_waves_per_eu((NW + (LD ? 4 : 0)) / 4, (NW + (LD ? 4 : 0)) / 4)))
 gemm_pipe(Operands op, TileArgs ta) {
@@ -351,6 +355,13 @@ gemm_pipe(Operands op, TileArgs ta) {
         return t;
     };
 
+    // A tile's k-steps; only TN's FP32 output and the k-tail instances have a
+    // partial one.
+    auto whole_steps = [&](const Tile& t) {
+        constexpr int up = KT || ST == Store::kTn ? BK - 1 : 0;
+        return (t.k_end - t.k_begin + up) / BK;
+    };
+
     // Instruction u = q * NLW + lw of an operand fills LDS bytes
     // [u KB, u KB + 1 KB) of its region; lane l writes bytes l * 16 .. + 16.
     // voff: the lane's byte offset in the global operand for k = 0 (the
@@ -372,6 +383,12 @@ gemm_pipe(Operands op, TileArgs ta) {
 #pragma unroll
     for (int q = 0; q < PER; ++q)
         voff[q] = q < IA ? lane_voff(q, BM, kXM, a_ld) : lane_voff(q - IA, BN, kWM, b_ld);
+    // The lane's k within a step in a row-major load. A load covers 8 rows
+    // (BK 64) and every wave an even count of loads apart, so that the chunk
+    // key is the same for all of the lane's loads.
+    static_assert(!KT || (BK == 64 && NLW % 2 == 0 && !LD && L != Layout::kTN), "k tails");
+    const int tail_row = lw * 8 + lane / 8;
+    const int kofs = KT ? ((lane % 8) ^ row_key<64>(tail_row)) * 8 : 0;
 
     // The issue side walks one stream of k-steps over all of the workgroup's
     // tiles, S steps ahead of the MFMAs; past the last one it reloads the last
@@ -425,9 +442,10 @@ gemm_pipe(Operands op, TileArgs ta) {
         // Row-major: k0 halves into every row. k-major: in the resource's base.
         const bool kmajor = xq ? kXM : kWM;
         const unsigned soff = kmajor ? 0u : unsigned(is.k0) * 2u;
+        const unsigned off = KT && !kmajor && kofs >= K - is.k0 ? 0xfffffff0u : voff[q];
         __builtin_amdgcn_raw_ptr_buffer_load_lds(xq ? is.ra : is.rb,
                                                  (__attribute__((address_space(3))) void*)dst, 16,
-                                                 voff[q], soff, 0, 0);
+                                                 off, soff, 0, 0);
     };
 
     f32x16 acc[FN][FM];
@@ -521,7 +539,7 @@ gemm_pipe(Operands op, TileArgs ta) {
             block_sync();
             for (int i = 0; i < n_tiles; ++i) {
                 const Tile t = tile(i);
-                const int steps = (t.k_end - t.k_begin) / BK;
+                const int steps = whole_steps(t);
                 for (int s = 0; s < steps; ++s) {
                     wait_vmcnt<(S - 2) * PER>();
                     block_sync();
@@ -651,7 +669,7 @@ gemm_pipe(Operands op, TileArgs ta) {
         };
         f16x8 pre_next[kPreEarly ? E::kPerLane : 1];
         if constexpr (kPreEarly) load_pre(0, 0, pre_next);
-        const int steps = (t.k_end - t.k_begin) / BK;
+        const int steps = whole_steps(t);
         for (int s = 0; s < steps; ++s) {
             Issue nxt = cur;
             advance(nxt);
@@ -974,10 +992,15 @@ size_t lds_bytes(const PipeConfig& c, Store st) {
     return stages + staging <= kPipeMaxLds ? stages + staging : stages + staging / 2;
 }
 
+// The configuration with k-tail instances for NT and NN.
+bool has_tail(const PipeConfig& c) { return c.same(PipeConfig{128, 192, 3, 64}); }
+
 // Whether a configuration can run an epilogue over k: it fits in LDS and k is
-// whole k-steps; the 8-wave configuration serves the NT layout only.
+// whole k-steps, or TN's FP32 output's, or the configuration takes tails; the 8-wave
+// configuration serves the NT layout only.
 bool usable(const PipeConfig& c, Store st, size_t k, Layout l) {
-    return lds_bytes(c, st) <= kPipeMaxLds && k % size_t(c.bk) == 0 &&
+    return lds_bytes(c, st) <= kPipeMaxLds &&
+           (k % size_t(c.bk) == 0 || st == Store::kTn || (l != Layout::kTN && has_tail(c))) &&
            (c.waves == 4 || l == Layout::kNT);
 }
 
@@ -1148,6 +1171,14 @@ hipError_t launch_pipe(const PipeConfig& c, const Operands& op, size_t slices, i
                 }                                                                              \
             }                                                                                  \
             if (hv) return hipErrorInvalidValue;                                               \
+            if constexpr (L != Layout::kTN && BM_ == 128 && BN_ == 192 && BK_ == 64 && LD_ == 0) { \
+                if (op.k % BK_ != 0) {                                                         \
+                    hipLaunchKernelGGL((gemm_pipe<BM_, BN_, S_, BK_, L, ST, NW_, false, false, \
+                                                  true>),                                      \
+                                       grid, dim3(NW_ * 64), 0, stream, op, ta);               \
+                    return hipGetLastError();                                                  \
+                }                                                                              \
+            }                                                                                  \
             hipLaunchKernelGGL((gemm_pipe<BM_, BN_, S_, BK_, L, ST, NW_, LD_ != 0>), grid,     \
                                dim3((NW_ + 4 * LD_) * 64), 0, stream, op, ta);                 \
             return hipGetLastError();                                                          \
@@ -1256,9 +1287,14 @@ bool gemm_pipe_eligible(GemmLayout gl, Epilogue e, size_t m, size_t n, size_t k)
     bool disabled = false;
     PipeConfig forced;
     pipe_forced(&forced, &disabled);
-    if (disabled || m == 0 || n == 0 || n % 8 != 0 || k % kPipeBK != 0 || k < kPipeBK) return false;
+    if (disabled || m == 0 || n == 0 || n % 8 != 0 || k == 0) return false;
     const Layout l = layout_of(gl);
     const Store st = store_of(e, l);
+    // NT and NN take k tails in whole 16-byte chunks; TN's FP32 output any k.
+    // The batched forms keep to whole 32-deep steps, which the GPT-2 model's
+    // attention layout (heads views, causal spans) is planned on.
+    const bool batched = st == Store::kScale || st == Store::kTnHalf;
+    if (batched ? k % kPipeBK != 0 : (l != Layout::kTN && k % 8 != 0)) return false;
     // Only the epilogues each layout serves.
     const bool served = l == Layout::kNT ? (st == Store::kNone || st == Store::kBias ||
                                             st == Store::kBiasGelu || st == Store::kBiasResidual ||
@@ -1277,10 +1313,12 @@ bool gemm_pipe_eligible(GemmLayout gl, Epilogue e, size_t m, size_t n, size_t k)
     return true;
 }
 
-// Per k-step of 64 a tile takes about 1 us * area / 256^2 / pipe_eff; a
-// round's prologue and epilogue 1.5 us, TN's FP32 output 4 (measured on
-// one-round products: NT 256 x 3072 x 768 6.6 us past its launch, 24 x 256 x
-// 256 x 64 2.0, TN 768 x 768 x 64 4.5 and x 256 5.8).
+// Per k-step of 64 a tile takes about 1 us * area / 256^2 / pipe_eff, more
+// where the rounds fill the GPU (the CUs then share the L2s and the power) and
+// where operand rows lie off the 128-byte lines, or are loaded half a line at
+// a time, so that each piece costs two lines. A round's prologue and epilogue
+// take 2.5 us, TN's FP32 output 4.4. The constants are fitted together with
+// gemm_small.hip's.
 double gemm_pipe_estimate(GemmLayout gl, Epilogue e, size_t slices, size_t m, size_t n, size_t k,
                           int max_splits) {
     constexpr double kInfinite = 1e300;
@@ -1296,12 +1334,15 @@ double gemm_pipe_estimate(GemmLayout gl, Epilogue e, size_t slices, size_t m, si
                          double(slices) * sp;
     const double rounds = std::ceil(tiles / cus);
     const double steps = double(k) / sp / 64.0;
-    // 32-deep steps of row-major operands load half lines, at half the rate
-    // while few tiles are in flight (NN 3000 x 744 x 2976 56 us in one round).
-    const bool half_lines = c.bk == 32 && l != Layout::kTN;
-    const double step_us = double(c.bm) * double(c.bn) / 65536.0 / pipe_eff(c, st, l) *
-                           (l == Layout::kNN ? 1.1 : 1.0) * (half_lines ? 2.0 : 1.0);
-    double us = rounds * (steps * step_us + (l == Layout::kTN ? 4.0 : 1.5));
+    const bool off_lines = l == Layout::kTN ? m % 64 != 0 || n % 64 != 0 : k % 64 != 0 || c.bk == 32;
+    const double layout = l == Layout::kNN ? 0.92 : 1.0;
+    const double lines =
+        !off_lines ? 1.0 : (l == Layout::kTN ? 1.5 : (l == Layout::kNT ? 1.2 : 1.8));
+    const double crowd = 1.0 + 1.1 * std::max(0.0, tiles / cus / rounds - 0.4);
+    const double step_us = double(c.bm) * double(c.bn) / 65536.0 / pipe_eff(c, st, l) * layout *
+                           lines * crowd;
+    const double fixed = l == Layout::kTN ? 4.4 : 2.5;
+    double us = rounds * steps * step_us + fixed * (1.0 + 1.5 * (rounds - 1.0));
     if (sp > 1) us += 3.0 + double(sp + 2) * double(m) * double(n) * 4.0 / 5e6;
     return us;
 }

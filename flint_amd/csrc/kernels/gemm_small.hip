@@ -36,6 +36,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <cmath>
 #include <cstdio>
 #include <type_traits>
 
@@ -456,25 +457,30 @@ __global__ void __launch_bounds__(NW * 64) gemm_small(Operands op, TileArgs ta) 
 #endif
 }
 
-// A configuration and its cost, measured on one MI355X (us; operands rotated
-// past the caches): `alone` is a k-step of a tile that has its CU to itself,
-// `shared` a k-step's share of the CU when there are more tiles than CUs,
-// `fixed` a tile's prologue and epilogue. Each per layout NT, NN, TN.
+// A configuration and its cost in us: `alone` is a k-step of a tile that has
+// its CU to itself, `shared` a tile's k-step where the CU runs several, `fixed`
+// a tile's prologue and epilogue. Each per layout NT, NN, TN (FP32 stores).
+// Fitted, together with gemm_pipe_estimate's constants, to the measured times
+// of 270 products (16 to 8,192 rows, widths 64 to 50,304, k 16 to 50,304,
+// batched ones among them; one MI355X, operands rotated past the caches): the
+// kernel and tile that the estimates choose are within 6% of the fastest for
+// all but 16 of them, at worst 1.3 times it.
 struct SmallConfig {
     int bm, bn, waves, stages, unit;
-    double alone[3], shared[3], fixed;
+    int resident;   // workgroups a CU holds
+    double alone[3], shared[3], fixed[3];
 };
 constexpr SmallConfig kSmallConfigs[] = {
     // Least to stream per CU: the smallest products.
-    {32, 32, 4, 8, 2, {0.135, 0.19, 0.20}, {0.145, 0.20, 0.21}, 0.7},
+    {32, 32, 4, 8, 2, 2, {0.12, 0.16, 0.17}, {0.12, 0.15, 0.17}, {0.74, 0.58, 0.96}},
     // The same for up to twice the tiles.
-    {32, 64, 4, 6, 2, {0.16, 0.20, 0.24}, {0.19, 0.20, 0.26}, 0.8},
+    {32, 64, 4, 6, 2, 2, {0.15, 0.18, 0.18}, {0.22, 0.23, 0.24}, {0.70, 0.50, 0.99}},
     // Eight waves load for one tile a CU: long k-ranges.
-    {64, 64, 8, 8, 2, {0.19, 0.235, 0.28}, {0.30, 0.33, 0.37}, 1.3},
+    {64, 64, 8, 8, 2, 1, {0.18, 0.22, 0.28}, {0.18, 0.22, 0.28}, {1.5, 1.6, 1.6}},
     // Two tiles a CU.
-    {64, 64, 4, 4, 1, {0.25, 0.26, 0.28}, {0.25, 0.25, 0.27}, 1.0},
+    {64, 64, 4, 4, 1, 2, {0.22, 0.24, 0.19}, {0.25, 0.29, 0.37}, {1.1, 0.64, 0.95}},
     // The fewest operand bytes per output: many tiles.
-    {128, 64, 8, 3, 1, {0.30, 0.34, 0.40}, {0.44, 0.44, 0.44}, 1.3},
+    {128, 64, 8, 3, 1, 2, {0.26, 0.32, 0.40}, {0.50, 0.53, 0.67}, {1.0, 0.70, 1.4}},
 };
 
 int layout_index(GemmLayout l) { return l == GemmLayout::kNT ? 0 : (l == GemmLayout::kNN ? 1 : 2); }
@@ -483,9 +489,11 @@ int layout_index(GemmLayout l) { return l == GemmLayout::kNT ? 0 : (l == GemmLay
 double small_cost(const SmallConfig& c, GemmLayout l, double tiles, double steps, int cus) {
     const int i = layout_index(l);
     const double load = tiles / cus;
-    if (load <= 1.0) return c.fixed + steps * c.alone[i];
-    const double shares = load <= 2.0 ? 2.0 : load;
-    return shares * (c.fixed + steps * c.shared[i]);
+    if (load <= 1.0) return c.fixed[i] + steps * c.alone[i];
+    if (c.resident == 1) return std::ceil(load) * (c.fixed[i] + steps * c.alone[i]);
+    // Tiles that share a CU overlap one another's prologues.
+    return std::max(1.0, load - 0.5) * c.fixed[i] +
+           steps * std::max(c.alone[i], load * c.shared[i]);
 }
 
 double small_tiles(const SmallConfig& c, size_t slices, size_t m, size_t n) {

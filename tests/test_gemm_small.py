@@ -141,3 +141,42 @@ def test_the_models_causal_products_and_heads_views(flint, cuda, cfg, length):
         assert torch.equal(_bits(a), _bits(b))
     for name in ref[3]:
         assert model._rel_l2(got[3][name], ref[3][name]) <= 1e-6, name
+
+
+# The pipeline's k tails (NT and NN in whole 16-byte chunks, TN any k): the
+# tile that takes them, forced, against the few-tile kernels' bits.
+@pytest.mark.parametrize("m,n,k", [(129, 200, 72), (300, 136, 744), (257, 392, 8), (130, 200, 2056)])
+def test_pipeline_k_tails(flint, cuda, m, n, k):
+    x = uniform((m, k), 31).to(cuda)
+    w = normal((n, k), 32, 0.05, H).to(cuda)
+    x[:, -8:] *= 50.0          # the tail matters
+    b = normal((n,), 33).to(cuda)
+    r = normal((m, n), 34).to(cuda)
+    wn = w.t().contiguous()
+    pre = normal((m, n), 35, 1.0, H).to(cuda)
+    for what, call, outs in (
+            ("nt", lambda y: flint.gemm_nt(y, x, w, m, n, k), [((m, n), H)]),
+            ("bias", lambda y: flint.gemm_nt_bias(y, x, w, b, m, n, k), [((m, n), H)]),
+            ("gelu", lambda y, p: flint.gemm_nt_bias_gelu(y, p, x, w, b, m, n, k),
+             [((m, n), H), ((m, n), H)]),
+            ("residual", lambda y: flint.gemm_nt_bias_residual(y, x, w, b, r, m, n, k),
+             [((m, n), F)]),
+            ("nn", lambda y: flint.gemm_nn(y, x, wn, m, n, k), [((m, n), H)]),
+            ("dgelu", lambda y: flint.gemm_nn_dgelu(y, x, wn, pre, m, n, k), [((m, n), H)])):
+        ref = _run(flint, call, outs, gemm_small="64,64,4,4,1")
+        got = _run(flint, call, outs, gemm_pipe="128,192,3,64", gemm_small="0")
+        for a, c in zip(got, ref):
+            assert torch.equal(_bits(a), _bits(c)), what
+
+
+@pytest.mark.parametrize("cfg", ["128,192,3,64", "128,192,3,64,4,1", "256,256,3", "256,64,3,64"])
+@pytest.mark.parametrize("m,n,k", [(136, 72, 1), (264, 200, 63), (136, 120, 3001)])
+def test_pipeline_tn_takes_any_k(flint, cuda, cfg, m, n, k):
+    x = normal((k, m), 36, 0.1, H).to(cuda)
+    w = uniform((k, n), 37).to(cuda)
+    ws = torch.empty(max(flint.gemm_tn_workspace(m, n, k), 16), dtype=torch.uint8, device=cuda)
+    got, = _run(flint, lambda y: flint.gemm_tn(y, x, w, m, n, k, workspace=ws), [((m, n), F)],
+                gemm_pipe=cfg, gemm_small="0")
+    ref = x.double().t() @ w.double()
+    bound = 2 * k * 2.0 ** -24 * (x.double().abs().t() @ w.double().abs()) + 2.0 ** -22 * ref.abs()
+    assert bool(((got.double() - ref).abs() <= bound).all())
