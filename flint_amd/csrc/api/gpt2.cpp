@@ -639,6 +639,12 @@ flint_status linear_grads(const flint_gpt2& m, const Param& w, const Param& b, c
     int splits = 1;
     FLINT_HIP_CHECK(flint::launch_gemm_tn_split(w.grad, dy, x, w.rows, w.cols, m.rows, acc != 0,
                                                 m.tn_work, &splits, hs));
+    // Few rows: the weight gradient unsplit and the bias gradient in a launch
+    // of its own leave the finish nothing to do.
+    if (splits == 1 && flint::bias_gradient_one_launch(m.rows, b.cols)) {
+        FLINT_HIP_CHECK(flint::launch_bias_gradient(b.grad, dy, m.rows, b.cols, acc != 0, m.work, hs));
+        return flush_merge(m, st);
+    }
     FLINT_HIP_CHECK(flint::launch_bias_partials(m.work, dy, m.rows, b.cols, hs));
     // The finish also carries a LayerNorm backward's deferred merge.
     FLINT_HIP_CHECK(flint::launch_linear_grads_finish(w.grad, m.tn_work, w.rows, w.cols, splits,

@@ -25,6 +25,8 @@ enum class Tune : int {
     kAttnScores,    // "0": the model's scores and dP through the batched product
                     // and the softmax passes (no fused scores + softmax)
     kEmbScan,       // "0": the embedding backward's token rows through the sort
+    kSumsFew,       // "0": the bias gradient and LayerNorm backward's parameter
+                    // sums always by chunk partials and a finish launch
     kGemmSmall,     // "0": no few-tile GEMM kernels; "bm,bn,waves,stages,unit":
                     // that tile for every GEMM
     kCount

@@ -205,6 +205,8 @@ hipError_t launch_layernorm_backward(void* dx, void* dgamma, void* dbeta, const 
 hipError_t launch_params_merge(const ParamsMerge& merge, hipStream_t stream);
 hipError_t launch_bias_gradient(void* dbias, const void* dy, size_t rows, size_t cols,
                                 bool accumulate, void* workspace, hipStream_t stream);
+// Whether launch_bias_gradient takes this shape in one launch (no workspace).
+bool bias_gradient_one_launch(size_t rows, size_t cols);
 // The same two passes with the partials in the library's per-device scratch
 // array (kBiasGradientScratchBytes; no allocation). Sizes whose partials do
 // not fit return hipErrorInvalidValue.

@@ -277,6 +277,88 @@ column_finish(float* __restrict__ out, const float* __restrict__ partial, size_t
     finish_quad(out, partial, chunks, cols, accumulate, quad, threadIdx.x & 31);
 }
 
+// finish_quad's merge of up to kFewChunks chunks, one column a lane, from LDS:
+// lane l of the 32-lane butterfly holds chunk l and the others nothing, so
+// lane 0's steps over xor 16 and 8 merge empty sums, and xor 4, 2 and 1 leave
+// the tree below (comp_merge is symmetric).
+constexpr int kFewChunks = 8;
+template <int COLS>
+using ChunkColumns = float[kFewChunks][COLS];
+template <int COLS>
+__device__ __forceinline__ float merge_few_chunks(const ChunkColumns<COLS>& sums,
+                                                  const ChunkColumns<COLS>& errs, int chunks, int c) {
+    Comp t[kFewChunks];
+#pragma unroll
+    for (int k = 0; k < kFewChunks; ++k) {
+        if (k < chunks) comp_merge(t[k], sums[k][c], errs[k][c]);
+        comp_merge(t[k], 0.0f, 0.0f);
+        comp_merge(t[k], 0.0f, 0.0f);
+    }
+#pragma unroll
+    for (int off = kFewChunks / 2; off > 0; off /= 2)
+#pragma unroll
+        for (int k = 0; k < off; ++k) comp_merge(t[k], t[k + off].sum, t[k + off].error);
+    return comp_value(t[0]);
+}
+
+// The bias gradient of up to 128 / COLS chunks in one launch: column_partials'
+// sums of all chunks of COLS columns at once (a wave holds one phase of
+// 64 / COLS chunks, waves 8 .. 15 the chunks after those of waves 0 .. 7), and
+// column_finish's merge of them from LDS. What bounds it is latency, of one
+// round of loads and of the sums' chain; the second launch for a few KB of
+// partials cost as much again. One MI355X, launches included: 256 x 768 7.1 ->
+// 4.0 us, 512 x 2304 7.2 -> 4.7, 1000 x 800 7.3 -> 4.8, 2048 x 768 7.2 -> 6.7;
+// 2048 x 3072, whose bytes count, 8.7 -> 11.1 (two launches there).
+template <int COLS>
+__global__ void __launch_bounds__(2 * kPhases * 64)
+bias_gradient_few(float* __restrict__ out, const _Float16* __restrict__ dy, size_t rows, int cols,
+                  int chunks, int accumulate) {
+    constexpr int kPer = kChunkRows / kPhases;
+    constexpr int kPerWave = 64 / COLS;   // chunks a wave holds
+    __shared__ float sums[kPhases - 1][2][64];
+    __shared__ float errs[kPhases - 1][2][64];
+    __shared__ ChunkColumns<COLS> chunk_sums, chunk_errs;
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(int(threadIdx.x >> 6));
+    const int ph = wave & (kPhases - 1), half = wave / kPhases;
+    const int c = lane % COLS;
+    const int chunk = half * kPerWave + lane / COLS;
+    const int col = int(blockIdx.x) * COLS + c;
+    const bool live = col < cols;
+    const size_t first = size_t(chunk) * kChunkRows;
+    const int count = first < rows ? int(min(rows - first, size_t(kChunkRows))) : 0;
+    const int n = count > ph ? (count - ph + kPhases - 1) / kPhases : 0;
+    // Rows past the chunk's end and columns past cols load element 0 and are
+    // never added, as in column_partials.
+    const size_t step = size_t(kPhases) * size_t(cols);
+    size_t at = (first + ph) * size_t(cols) + col;
+    _Float16 d[kPer];
+#pragma unroll
+    for (int k = 0; k < kPer; ++k) {
+        d[k] = dy[k < n && live ? at : 0];
+        at += step;
+    }
+    Comp acc;
+#pragma unroll
+    for (int k = 0; k < kPer; ++k)
+        if (k < n) comp_add(acc, float(d[k]));
+    if (ph > 0) {
+        sums[ph - 1][half][lane] = acc.sum;
+        errs[ph - 1][half][lane] = acc.error;
+    }
+    __syncthreads();
+    if (ph == 0 && chunk < chunks) {
+#pragma unroll
+        for (int o = 0; o < kPhases - 1; ++o) comp_merge(acc, sums[o][half][lane], errs[o][half][lane]);
+        chunk_sums[chunk][c] = acc.sum;
+        chunk_errs[chunk][c] = acc.error;
+    }
+    __syncthreads();
+    if (threadIdx.x >= COLS || !live) return;
+    const float r = merge_few_chunks<COLS>(chunk_sums, chunk_errs, chunks, c);
+    out[col] = accumulate ? add_rn(out[col], r) : r;
+}
+
 // A merge of two column-partial sets (a LayerNorm's dbeta into out0, dgamma
 // into out1).
 struct ColumnFinish {
@@ -321,20 +403,24 @@ linear_grads_finish(float* __restrict__ dw, const float* __restrict__ dw_partial
 // column_partials<true, 1>, in their order, into part0 and part1. The dx
 // kernel launched after it merges them (ColumnFinish).
 // Units b = first, first + stride, ... < blocks (chunk x 64 columns each) of a
-// kPhases * 64-thread workgroup.
+// kPhases * 64-thread workgroup. MERGED (rows of one chunk): the sums go
+// through finish_quad's merge of a single chunk -- into an empty sum, then five
+// empty lanes' -- straight into out0 and out1.
+template <bool MERGED>
 __device__ __forceinline__ void partials2_units(float* part0, float* part1,
                                                 const _Float16* __restrict__ dy,
                                                 const float* __restrict__ x,
                                                 const float* __restrict__ mean,
                                                 const float* __restrict__ rstd, size_t rows,
                                                 int cols, size_t chunks, size_t blocks,
-                                                size_t first, size_t stride_b) {
+                                                size_t first_unit, size_t stride_b,
+                                                const ColumnFinish& merge) {
     constexpr int kPer = kChunkRows / kPhases;
     __shared__ float sums[2][kPhases - 1][64];
     __shared__ float errs[2][kPhases - 1][64];
     const int lane = threadIdx.x & 63;
     const int ph = __builtin_amdgcn_readfirstlane(int(threadIdx.x >> 6));
-    for (size_t b = first; b < blocks; b += stride_b) {
+    for (size_t b = first_unit; b < blocks; b += stride_b) {
         const int tile = int(b / chunks);
         const size_t chunk = b - size_t(tile) * chunks;
         const size_t first = chunk * kChunkRows;
@@ -385,9 +471,18 @@ __device__ __forceinline__ void partials2_units(float* part0, float* part1,
 #pragma unroll
                 for (int o = 0; o < kPhases - 1; ++o)
                     comp_merge(acc[u], sums[u][o][lane], errs[u][o][lane]);
-                float* part = u == 0 ? part0 : part1;
-                part[chunk * 2 * cols + col] = acc[u].sum;
-                part[(chunk * 2 + 1) * cols + col] = acc[u].error;
+                if constexpr (MERGED) {
+                    Comp t;
+                    comp_merge(t, acc[u].sum, acc[u].error);
+                    for (int k = 0; k < 5; ++k) comp_merge(t, 0.0f, 0.0f);
+                    const float r = comp_value(t);
+                    float* out = u == 0 ? merge.out0 : merge.out1;
+                    out[col] = merge.accumulate ? add_rn(out[col], r) : r;
+                } else {
+                    float* part = u == 0 ? part0 : part1;
+                    part[chunk * 2 * cols + col] = acc[u].sum;
+                    part[(chunk * 2 + 1) * cols + col] = acc[u].error;
+                }
             }
         }
         __syncthreads();
@@ -399,8 +494,8 @@ column_partials2(float* part0, float* part1, const _Float16* __restrict__ dy,
                  const float* __restrict__ x, const float* __restrict__ mean,
                  const float* __restrict__ rstd, size_t rows, int cols, size_t chunks,
                  size_t blocks) {
-    partials2_units(part0, part1, dy, x, mean, rstd, rows, cols, chunks, blocks, blockIdx.x,
-                    gridDim.x);
+    partials2_units<false>(part0, part1, dy, x, mean, rstd, rows, cols, chunks, blocks, blockIdx.x,
+                           gridDim.x, ColumnFinish{});
 }
 
 hipError_t launch_partials(float* partial, const void* dy, size_t rows, size_t cols,
@@ -535,17 +630,19 @@ layernorm_backward_dx(float* __restrict__ dx, const _Float16* __restrict__ dy,
 // per half-wave (layernorm_backward_dx's), so that the latency-bound partials
 // overlap the bandwidth-bound rows; ln_params_finish merges the partials
 // after it. The same arithmetic in the same order as the two-launch path.
-template <int PPL>
+// MERGED (one chunk of rows): the partials workgroups finish dbeta and dgamma
+// themselves, with no launch after it.
+template <int PPL, bool MERGED>
 __global__ void __launch_bounds__(kPhases * 64)
 layernorm_backward_fused(float* part0, float* part1, float* __restrict__ dx,
                          const _Float16* __restrict__ dy, const float* __restrict__ x,
                          const float* __restrict__ mean, const float* __restrict__ rstd,
                          const float* __restrict__ gamma, size_t rows, int cols, size_t chunks,
                          size_t items, unsigned units, int accumulate,
-                         _Float16* __restrict__ dx_half) {
+                         _Float16* __restrict__ dx_half, ColumnFinish merge) {
     if (blockIdx.x < units) {
-        partials2_units(part0, part1, dy, x, mean, rstd, rows, cols, chunks, items, blockIdx.x,
-                        units);
+        partials2_units<MERGED>(part0, part1, dy, x, mean, rstd, rows, cols, chunks, items,
+                                blockIdx.x, units, merge);
         return;
     }
     dx_rows<PPL, kPhases * 2>(dx, dy, x, mean, rstd, gamma, rows, cols, accumulate, dx_half,
@@ -912,8 +1009,27 @@ hipError_t launch_params_merge(const ParamsMerge& merge, hipStream_t stream) {
     return hipGetLastError();
 }
 
+bool bias_gradient_one_launch(size_t rows, size_t cols) {
+    // Measured even at 1024 x 3072 (7.1 against 7.5 us), see bias_gradient_few.
+    constexpr size_t kMostValues = size_t{4} << 20;
+    return rows <= size_t(kFewChunks) * kChunkRows && rows * cols <= kMostValues &&
+           !tuning_off(Tune::kSumsFew);
+}
+
 hipError_t launch_bias_gradient(void* dbias, const void* dy, size_t rows, size_t cols,
                                 bool accumulate, void* workspace, hipStream_t stream) {
+    if (bias_gradient_one_launch(rows, cols)) {
+        const size_t chunks = (rows + kChunkRows - 1) / kChunkRows;
+        auto few = [&](auto kernel, size_t columns) {
+            hipLaunchKernelGGL(kernel, dim3(unsigned((cols + columns - 1) / columns)),
+                               dim3(2 * kPhases * 64), 0, stream, static_cast<float*>(dbias),
+                               static_cast<const _Float16*>(dy), rows, int(cols), int(chunks),
+                               accumulate ? 1 : 0);
+        };
+        if (chunks <= 2) few(bias_gradient_few<64>, 64);
+        else few(bias_gradient_few<16>, 16);
+        return hipGetLastError();
+    }
     if (hipError_t e = launch_partials(static_cast<float*>(workspace), dy, rows, cols, stream);
         e != hipSuccess) {
         return e;
@@ -949,20 +1065,29 @@ hipError_t launch_layernorm_backward(void* dx, void* dgamma, void* dbeta, const 
     // the partials, then dx with the merge; the same bits).
     const bool fused = pieces <= 256 && !tuning_off(Tune::kLnFused);
     if (fused) {
+        // One chunk: merged in the same launch (256 x 768 10.8 -> 7.2 us). Two
+        // and more, one after the other in a workgroup, took 5 us a chunk
+        // against the merge launch's 3.5 (512 x 768 11.7 against 9.9).
+        const bool merged = chunks == 1 && !tuning_off(Tune::kSumsFew);
         const size_t units = std::min<size_t>(items, 1u << 20);
         const size_t row_blocks = std::min<size_t>((rows + 15) / 16, kMaxBlocks);
         const dim3 grid(unsigned(units + row_blocks));
 #define FLINT_LNF(PPL)                                                                         \
-    hipLaunchKernelGGL(layernorm_backward_fused<PPL>, grid, dim3(kPhases * 64), 0, stream,     \
-                       part0, part1, dxf, dyh, xf, mf, rf, gf, rows, c, chunks, items,         \
-                       unsigned(units), acc, dxh)
-        if (pieces <= 32) FLINT_LNF(1);
-        else if (pieces <= 64) FLINT_LNF(2);
-        else if (pieces <= 96) FLINT_LNF(3);
-        else if (pieces <= 128) FLINT_LNF(4);
-        else FLINT_LNF(8);
+    if (merged)                                                                                \
+        hipLaunchKernelGGL((layernorm_backward_fused<PPL, true>), grid, dim3(kPhases * 64), 0, \
+                           stream, part0, part1, dxf, dyh, xf, mf, rf, gf, rows, c, chunks,    \
+                           items, unsigned(units), acc, dxh, finish);                          \
+    else                                                                                       \
+        hipLaunchKernelGGL((layernorm_backward_fused<PPL, false>), grid, dim3(kPhases * 64), 0, \
+                           stream, part0, part1, dxf, dyh, xf, mf, rf, gf, rows, c, chunks,    \
+                           items, unsigned(units), acc, dxh, finish)
+        if (pieces <= 32) { FLINT_LNF(1); }
+        else if (pieces <= 64) { FLINT_LNF(2); }
+        else if (pieces <= 96) { FLINT_LNF(3); }
+        else if (pieces <= 128) { FLINT_LNF(4); }
+        else { FLINT_LNF(8); }
 #undef FLINT_LNF
-        if (hipError_t e = hipGetLastError(); e != hipSuccess) return e;
+        if (hipError_t e = hipGetLastError(); e != hipSuccess || merged) return e;
         const ParamsMerge merge{static_cast<float*>(dbeta), static_cast<float*>(dgamma), part0,
                                 part1, chunks, c, accumulate_params ? 1 : 0};
         if (deferred != nullptr) {
