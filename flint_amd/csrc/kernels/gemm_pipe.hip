@@ -1317,7 +1317,7 @@ bool gemm_pipe_eligible(GemmLayout gl, Epilogue e, size_t m, size_t n, size_t k)
 // where the rounds fill the GPU (the CUs then share the L2s and the power) and
 // where operand rows lie off the 128-byte lines, or are loaded half a line at
 // a time, so that each piece costs two lines. A round's prologue and epilogue
-// take 2.5 us, TN's FP32 output 4.4. The constants are fitted together with
+// take 2.7 to 2.8 us, TN's FP32 output 4.6. The constants are fitted together with
 // gemm_small.hip's.
 double gemm_pipe_estimate(GemmLayout gl, Epilogue e, size_t slices, size_t m, size_t n, size_t k,
                           int max_splits) {
@@ -1335,14 +1335,14 @@ double gemm_pipe_estimate(GemmLayout gl, Epilogue e, size_t slices, size_t m, si
     const double rounds = std::ceil(tiles / cus);
     const double steps = double(k) / sp / 64.0;
     const bool off_lines = l == Layout::kTN ? m % 64 != 0 || n % 64 != 0 : k % 64 != 0 || c.bk == 32;
-    const double layout = l == Layout::kNN ? 0.92 : 1.0;
+    const double layout = l == Layout::kNN ? 0.906 : 1.0;
     const double lines =
-        !off_lines ? 1.0 : (l == Layout::kTN ? 1.5 : (l == Layout::kNT ? 1.2 : 1.8));
-    const double crowd = 1.0 + 1.1 * std::max(0.0, tiles / cus / rounds - 0.4);
+        !off_lines ? 1.0 : (l == Layout::kNN ? 1.53 : (l == Layout::kNT ? 1.34 : 1.5));
+    const double crowd = 1.0 + 1.38 * std::max(0.0, tiles / cus / rounds - 0.4);
     const double step_us = double(c.bm) * double(c.bn) / 65536.0 / pipe_eff(c, st, l) * layout *
                            lines * crowd;
-    const double fixed = l == Layout::kTN ? 4.4 : 2.5;
-    double us = rounds * steps * step_us + fixed * (1.0 + 1.5 * (rounds - 1.0));
+    const double fixed = l == Layout::kTN ? 4.56 : (l == Layout::kNT ? 2.81 : 2.68);
+    double us = rounds * steps * step_us + fixed * (1.0 + 1.34 * (rounds - 1.0));
     if (sp > 1) us += 3.0 + double(sp + 2) * double(m) * double(n) * 4.0 / 5e6;
     return us;
 }

@@ -6,14 +6,16 @@
 // one CU's load rate. What bounds such a product is the bytes that one CU has
 // to stream (its tile's two operand strips) and the latency of the first of
 // them, so the tile here is as small as the MFMA's 32 x 32 allows:
-//  * 256 threads. WM x WN of the four waves each own one 32 x 32 block; all
-//    four issue the operand loads (a CU's load rate grows with the waves that
-//    issue: one wave alone reached a quarter of it), so a 32 x 32 tile has one
-//    MFMA wave and three that only load.
+//  * WM x WN waves each own one 32 x 32 block. Either they issue the operand
+//    loads as well, or (LD) four more waves do: a load holds its wave for
+//    about 33 cycles, as long as an MFMA takes, so that on a CU with one tile
+//    the MFMA wave's own loads cost it half its time (NT 256 x 768 x 3072 9.6
+//    -> 7.4 us with the loader waves, NN 11.3 -> 9.3; with eight of them 7.8).
+//    Where several tiles share a CU the extra waves only get in the way.
 //  * k-steps of 64 through S LDS stages by direct-to-LDS buffer loads, S steps
-//    in flight, one barrier a step. The fragments of step s + 1 are read
-//    while step s's MFMAs run, which also frees step s's stage for the load
-//    of step s + S at the same barrier.
+//    in flight, in groups of U steps with one barrier each. The fragments of
+//    the next group are read while a group's MFMAs run, which also frees its
+//    stages for the loads of the group S / U further on at the same barrier.
 //  * Each 32 x 32 block is one chain of v_mfma_f32_32x32x16_f16 over k in
 //    ascending order from a zero accumulator, as in the other GEMM kernels:
 //    the same sums, bit for bit, whichever kernel a shape runs on.
@@ -23,16 +25,18 @@
 //  * Ragged sizes: rows and columns past the operands read zeros or values
 //    that only reach outputs that are not stored; a k tail (k % 64) reads
 //    zeros from both operands.
-//  * Larger tiles (32 x 64 to 128 x 64, up to eight waves) take over as the
-//    tile count passes the CUs, until gemm_pipe.hip's tiles fill the GPU:
-//    gemm_small_plan compares both by their estimated times.
+//  * Larger tiles (32 x 64 to 128 x 64) take over as the tile count passes the
+//    CUs, until gemm_pipe.hip's tiles fill the GPU: gemm_small_plan compares
+//    all of them by their estimated times.
 // Measured (one MI355X, operands rotated past the caches, launch included,
-// before -> after): NT 64 x 768 x 3072 22.5 -> 9.4 us, 256 x 768 x 768 9.6 ->
-// 4.6, 1024 x 768 x 3072 25 -> 12.9; NN 256 x 768 x 50304 518 -> 178; TN 768 x
-// 768 x 256 9.1 -> 4.8; ragged NT 1000 x 200 x 800 14.0 -> 5.0, TN 768 x 768 x
-// 1000 60 -> 8.0. A tile's k-step takes 0.14 to 0.3 us: at 32 x 32 four
-// dependent MFMAs (about 150 cycles) and a barrier every second step, at 64 x
-// 64 the 32 KB of fragment reads (about 110 B a cycle).
+// against the kernels before these): NT 64 x 768 x 3072 22.4 -> 7.2 us, 256 x
+// 768 x 768 9.5 -> 4.6, 1024 x 768 x 3072 25 -> 12.2; NN 256 x 768 x 50304 518
+// -> 177; TN 768 x 768 x 256 9.0 -> 4.9; ragged NT 1000 x 200 x 800 14.0 ->
+// 4.6, TN 768 x 768 x 1000 60 -> 7.2. What bounds a tile alone on its CU: the
+// chain of dependent MFMAs (32 cycles each, 4 a k-step and block) and one
+// exposed LDS read per group; with the operand loads returning nothing at all
+// it takes as long. With several tiles a CU, the direct-to-LDS load rate
+// (about 32 B a cycle with four waves) and the fragment reads.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -66,7 +70,7 @@ __device__ __forceinline__ float settled(float x) {
     return x;
 }
 
-template <int WM, int WN, int NW, int S, int U, Layout L, Store ST, bool HV = false>
+template <int WM, int WN, int NW, int S, int U, bool LD, Layout L, Store ST, bool HV = false>
 __global__ void __launch_bounds__(NW * 64) gemm_small(Operands op, TileArgs ta) {
     // The host pass only needs a kernel to emit a launch stub for.
 #if defined(__HIP_DEVICE_COMPILE__)
@@ -84,8 +88,9 @@ __global__ void __launch_bounds__(NW * 64) gemm_small(Operands op, TileArgs ta) 
         ST == Store::kBias || ST == Store::kBiasGelu || ST == Store::kBiasResidual;
     constexpr bool kF32 = ST == Store::kBiasResidual || ST == Store::kTn;
     // A step's 1 KB loads, x's first, dealt to the waves in turn.
-    constexpr int kLoadsA = BM / 8, kLoads = (BM + BN) / 8, PER = kLoads / NW;
-    static_assert(kLoads % NW == 0 && S * PER < 64, "whole loads per wave, vmcnt range");
+    constexpr int NL = LD ? NW - WM * WN : NW;   // waves that load
+    constexpr int kLoadsA = BM / 8, kLoads = (BM + BN) / 8, PER = kLoads / NL;
+    static_assert(kLoads % NL == 0 && S * PER < 64, "whole loads per wave, vmcnt range");
     constexpr int kGroupLoads = U * PER;
     constexpr int kStage = (BM + BN) * kStep;
     constexpr int kLd = BN + 4;                       // staged sums: floats a row
@@ -96,6 +101,8 @@ __global__ void __launch_bounds__(NW * 64) gemm_small(Operands op, TileArgs ta) 
     const int lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int m = op.m, n = op.n, K = op.k;
+    const bool loads = !LD || wave >= WM * WN;
+    const int lw = LD ? max(wave - WM * WN, 0) : wave;   // among the loading waves
     const bool split = ST == Store::kTn && op.partials != nullptr;
 
     // ---- this workgroup's tile
@@ -141,12 +148,12 @@ __global__ void __launch_bounds__(NW * 64) gemm_small(Operands op, TileArgs ta) 
     const size_t a_bytes = kXM ? (size_t(K) * m - m0) * 2 : size_t(min(BM, m - m0)) * K * 2;
     const size_t b_bytes = kWM ? (size_t(K - 1) * b_ld + n - n0) * 2
                                : size_t(min(BN, n - n0)) * K * 2;
-    // Load v = q NW + wave of a step fills LDS bytes [v KB, v KB + 1 KB) of its
+    // Load v = q NL + lw of a step fills LDS bytes [v KB, v KB + 1 KB) of its
     // stage (x's region, then w's); lane l writes bytes 16 l .. + 15 of it.
     unsigned voff[PER];
     int kofs[PER];   // row-major: the lane's k within a step
     auto of_x = [&](int q) {
-        return kLoadsA % NW == 0 ? q < kLoadsA / NW : q * NW + wave < kLoadsA;
+        return kLoadsA % NL == 0 ? q < kLoadsA / NL : q * NL + lw < kLoadsA;
     };
     auto place = [&](int q, bool kmajor, int rows, int u, int ld) {
         if (kmajor) {
@@ -165,7 +172,7 @@ __global__ void __launch_bounds__(NW * 64) gemm_small(Operands op, TileArgs ta) 
     };
 #pragma unroll
     for (int q = 0; q < PER; ++q) {
-        const int v = q * NW + wave;
+        const int v = q * NL + lw;
         if (of_x(q)) place(q, kXM, BM, v, a_ld);
         else place(q, kWM, BN, v - kLoadsA, b_ld);
     }
@@ -173,6 +180,7 @@ __global__ void __launch_bounds__(NW * 64) gemm_small(Operands op, TileArgs ta) 
     // Loads step k0 into stage st. Steps past the last one load nothing (an
     // empty resource), so that every wait counts the same loads.
     auto issue = [&](int k0, int st) {
+        if (!loads) return;
         const bool live = k0 < k_end;
         const size_t ka = kXM ? size_t(k0) * a_ld : 0, kb = kWM ? size_t(k0) * b_ld : 0;
         const auto ra = __builtin_amdgcn_make_buffer_rsrc(
@@ -182,7 +190,7 @@ __global__ void __launch_bounds__(NW * 64) gemm_small(Operands op, TileArgs ta) 
         const int left = k_end - k0;
 #pragma unroll
         for (int q = 0; q < PER; ++q) {
-            const int v = q * NW + wave;
+            const int v = q * NL + lw;
             lds_half* dst = (lds_half*)(lds + st * kStage + v * 512);
             auto load = [&](const auto& rsrc, bool kmajor) {
                 const unsigned off = kmajor || kofs[q] < left ? voff[q] : kOutside;
@@ -288,25 +296,30 @@ __global__ void __launch_bounds__(NW * 64) gemm_small(Operands op, TileArgs ta) 
     // Waits for a step's fragments. The empty asm uses the transposing reads'
     // registers, so that they stay theirs while the reads are in flight, also
     // where nothing uses the values (after the last step).
-    auto wait_frags = [&](const XFrag (&x)[4], const WFrag (&w)[4]) {
+    auto wait_frags = [&](const XFrag (&x)[4 * U], const WFrag (&w)[4 * U]) {
         __builtin_amdgcn_sched_barrier(0);
         __builtin_amdgcn_s_waitcnt(0xc07f);   // lgkmcnt(0)
         __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-        for (int kk = 0; kk < 4; ++kk) {
+        for (int kk = 0; kk < 4 * U; ++kk) {
             if constexpr (kXM) asm volatile("" ::"v"(x[kk].lo), "v"(x[kk].hi));
             if constexpr (kWM) asm volatile("" ::"v"(w[kk].lo), "v"(w[kk].hi));
         }
     };
-    XFrag xf[2][4];
-    WFrag wf[2][4];
-    auto read_frag = [&](int st, int kk, XFrag (&x)[4], WFrag (&w)[4]) {
-        const _Float16* s0 = lds + st * kStage;
-        if constexpr (kXM) x[kk] = frag_kmajor(s0, std::integral_constant<int, BM>{}, wm * 32, kk);
-        else x[kk] = frag_rowmajor(s0, wm * 32, kk);
+    // Fragments of a batch of kBatch steps: a whole group's, where groups have
+    // two steps, else a step's.
+    constexpr int kBatch = U, kFrags = 4 * kBatch;
+    XFrag xf[2][kFrags];
+    WFrag wf[2][kFrags];
+    // Fragment q of the batch whose first stage is st.
+    auto read_frag = [&](int st, int q, XFrag& x, WFrag& w) {
+        const _Float16* s0 = lds + (st + q / 4) * kStage;
+        const int kk = q % 4;
+        if constexpr (kXM) x = frag_kmajor(s0, std::integral_constant<int, BM>{}, wm * 32, kk);
+        else x = frag_rowmajor(s0, wm * 32, kk);
         if constexpr (kWM)
-            w[kk] = frag_kmajor(s0 + BM * kStep, std::integral_constant<int, BN>{}, wn * 32, kk);
-        else w[kk] = frag_rowmajor(s0 + BM * kStep, wn * 32, kk);
+            w = frag_kmajor(s0 + BM * kStep, std::integral_constant<int, BN>{}, wn * 32, kk);
+        else w = frag_rowmajor(s0 + BM * kStep, wn * 32, kk);
     };
 
     // Groups of U steps; a last group's steps past k_end add zeros.
@@ -318,59 +331,44 @@ __global__ void __launch_bounds__(NW * 64) gemm_small(Operands op, TileArgs ta) 
     block_sync();
     if (computes) {
 #pragma unroll
-        for (int kk = 0; kk < 4; ++kk) read_frag(0, kk, xf[0], wf[0]);
+        for (int q = 0; q < kFrags; ++q) read_frag(0, q, xf[0][q], wf[0][q]);
         wait_frags(xf[0], wf[0]);
     }
-    int st = 0;   // the stage of the step whose fragments are in registers
-    // One step: four MFMAs with the next step's fragment reads between them (a
-    // burst of reads before the MFMAs cost a third of the step). Before a
-    // group's last step reads on, the next group has landed for every wave,
-    // and every wave holds the last step's fragments, so the group's stages
-    // take the loads of the group S / U further on; its first MFMA runs under
-    // that barrier.
-    auto step = [&](bool last, XFrag (&x)[4], WFrag (&w)[4], XFrag (&xn)[4], WFrag (&wn_)[4]) {
-        auto mfma = [&](int kk) {
-            acc = __builtin_amdgcn_mfma_f32_32x32x16_f16(as_f16x8(w[kk]), as_f16x8(x[kk]), acc, 0, 0,
-                                                         0);
+    int st = 0;   // the first stage of the group whose fragments are in registers
+    // One group: its MFMAs with the next group's fragment reads between them
+    // (a burst of reads before the MFMAs cost a third of a step). Before the
+    // reads the next group has landed for every wave, and every wave holds
+    // this group's fragments, so its stages take the loads of the group S / U
+    // further on; the first MFMA runs under that barrier. One wait per group
+    // for the fragments: at the end of every step, it exposed the last read's
+    // latency each time.
+    auto group = [&](XFrag (&x)[kFrags], WFrag (&w)[kFrags], XFrag (&xn)[kFrags],
+                     WFrag (&wn_)[kFrags]) {
+        auto mfma = [&](int q) {
+            acc = __builtin_amdgcn_mfma_f32_32x32x16_f16(as_f16x8(w[q]), as_f16x8(x[q]), acc, 0, 0, 0);
             __builtin_amdgcn_sched_barrier(0);
         };
         if (computes) mfma(0);
-        if (last) {
-            wait_vmcnt<(S / U - 2) * kGroupLoads>();
-            block_sync();
+        wait_vmcnt<(S / U - 2) * kGroupLoads>();
+        block_sync();
 #pragma unroll
-            for (int j = 0; j < U; ++j, k0 += kStep) issue(k0, st - (U - 1) + j);
-        }
-        st = st + 1 == S ? 0 : st + 1;
+        for (int j = 0; j < U; ++j, k0 += kStep) issue(k0, st + j);
+        st = st + U == S ? 0 : st + U;
         if (computes) {
             __builtin_amdgcn_sched_barrier(0);
-            read_frag(st, 0, xn, wn_);
-            read_frag(st, 1, xn, wn_);
-            __builtin_amdgcn_sched_barrier(0);
-            mfma(1);
-            read_frag(st, 2, xn, wn_);
-            __builtin_amdgcn_sched_barrier(0);
-            mfma(2);
-            read_frag(st, 3, xn, wn_);
-            __builtin_amdgcn_sched_barrier(0);
-            mfma(3);
+            read_frag(st, 0, xn[0], wn_[0]);
+#pragma unroll
+            for (int q = 1; q < kFrags; ++q) {
+                read_frag(st, q, xn[q], wn_[q]);
+                __builtin_amdgcn_sched_barrier(0);
+                mfma(q);
+            }
             wait_frags(xn, wn_);
         }
     };
-    if constexpr (U == 1) {
-        for (int g = 0; g < groups; g += 2) {
-            step(true, xf[0], wf[0], xf[1], wf[1]);
-            if (g + 1 < groups) step(true, xf[1], wf[1], xf[0], wf[0]);
-        }
-    } else {
-        static_assert(U % 2 == 0, "fragment buffers alternate within a group");
-        for (int g = 0; g < groups; ++g) {
-#pragma unroll
-            for (int j = 0; j < U; j += 2) {
-                step(false, xf[0], wf[0], xf[1], wf[1]);
-                step(j + 2 == U, xf[1], wf[1], xf[0], wf[0]);
-            }
-        }
+    for (int g = 0; g < groups; g += 2) {
+        group(xf[0], wf[0], xf[1], wf[1]);
+        if (g + 1 < groups) group(xf[1], wf[1], xf[0], wf[0]);
     }
 
     // ---- epilogue: the sums through LDS (the stages, once every load into
@@ -463,24 +461,25 @@ __global__ void __launch_bounds__(NW * 64) gemm_small(Operands op, TileArgs ta) 
 // Fitted, together with gemm_pipe_estimate's constants, to the measured times
 // of 270 products (16 to 8,192 rows, widths 64 to 50,304, k 16 to 50,304,
 // batched ones among them; one MI355X, operands rotated past the caches): the
-// kernel and tile that the estimates choose are within 6% of the fastest for
-// all but 16 of them, at worst 1.3 times it.
+// kernel and tile that the estimates choose are within 7% of the fastest for
+// all but 10 of them, at worst 1.3 times it.
 struct SmallConfig {
     int bm, bn, waves, stages, unit;
     int resident;   // workgroups a CU holds
     double alone[3], shared[3], fixed[3];
 };
 constexpr SmallConfig kSmallConfigs[] = {
-    // Least to stream per CU: the smallest products.
-    {32, 32, 4, 8, 2, 2, {0.12, 0.16, 0.17}, {0.12, 0.15, 0.17}, {0.74, 0.58, 0.96}},
+    // Least to stream per CU, four loader waves beside the MFMA wave: the
+    // smallest products.
+    {32, 32, 5, 8, 2, 2, {0.052, 0.100, 0.172}, {0.128, 0.196, 0.195}, {1.0, 0.571, 1.02}},
     // The same for up to twice the tiles.
-    {32, 64, 4, 6, 2, 2, {0.15, 0.18, 0.18}, {0.22, 0.23, 0.24}, {0.70, 0.50, 0.99}},
-    // Eight waves load for one tile a CU: long k-ranges.
-    {64, 64, 8, 8, 2, 1, {0.18, 0.22, 0.28}, {0.18, 0.22, 0.28}, {1.5, 1.6, 1.6}},
+    {32, 64, 4, 6, 2, 2, {0.080, 0.170, 0.190}, {0.138, 0.185, 0.208}, {0.99, 0.291, 0.955}},
+    // One tile a CU, four loader waves: long k-ranges.
+    {64, 64, 8, 6, 2, 1, {0.098, 0.187, 0.193}, {0.250, 0.318, 0.308}, {1.35, 0.351, 1.15}},
     // Two tiles a CU.
-    {64, 64, 4, 4, 1, 2, {0.22, 0.24, 0.19}, {0.25, 0.29, 0.37}, {1.1, 0.64, 0.95}},
+    {64, 64, 4, 4, 1, 2, {0.178, 0.254, 0.235}, {0.234, 0.277, 0.314}, {1.03, 0.226, 0.776}},
     // The fewest operand bytes per output: many tiles.
-    {128, 64, 8, 3, 1, 2, {0.26, 0.32, 0.40}, {0.50, 0.53, 0.67}, {1.0, 0.70, 1.4}},
+    {128, 64, 8, 3, 1, 2, {0.263, 0.347, 0.410}, {0.393, 0.499, 0.630}, {1.12, 0.198, 0.645}},
 };
 
 int layout_index(GemmLayout l) { return l == GemmLayout::kNT ? 0 : (l == GemmLayout::kNN ? 1 : 2); }
@@ -490,10 +489,12 @@ double small_cost(const SmallConfig& c, GemmLayout l, double tiles, double steps
     const int i = layout_index(l);
     const double load = tiles / cus;
     if (load <= 1.0) return c.fixed[i] + steps * c.alone[i];
-    if (c.resident == 1) return std::ceil(load) * (c.fixed[i] + steps * c.alone[i]);
-    // Tiles that share a CU overlap one another's prologues.
+    if (c.resident == 1) return std::ceil(load) * (c.fixed[i] + steps * c.shared[i]);
+    // Tiles that share a CU overlap one another's prologues. The last round is
+    // as long as its fullest CU, but runs faster where the others are empty.
+    const double full = 0.5 * (load + std::ceil(load));
     return std::max(1.0, load - 0.5) * c.fixed[i] +
-           steps * std::max(c.alone[i], load * c.shared[i]);
+           steps * std::max(c.alone[i], full * c.shared[i]);
 }
 
 double small_tiles(const SmallConfig& c, size_t slices, size_t m, size_t n) {
@@ -535,17 +536,17 @@ hipError_t launch(const SmallPlan& c, const Operands& op, size_t slices, hipStre
     ta.group_m = 8;
     ta.split_len = c.split_len;
     const dim3 grid(unsigned(per * slices));
-#define FLINT_SMALL_CASE(BM_, BN_, NW_, S_, U_)                                                    \
+#define FLINT_SMALL_CASE(BM_, BN_, NW_, S_, U_, LD_)                                               \
     if (c.bm == BM_ && c.bn == BN_ && c.waves == NW_ && c.stages == S_ && c.unit == U_) {          \
-        hipLaunchKernelGGL((gemm_small<BM_ / 32, BN_ / 32, NW_, S_, U_, L, ST, HV>), grid,         \
+        hipLaunchKernelGGL((gemm_small<BM_ / 32, BN_ / 32, NW_, S_, U_, LD_, L, ST, HV>), grid,    \
                            dim3(NW_ * 64), 0, stream, op, ta);                                     \
         return hipGetLastError();                                                                  \
     }
-    FLINT_SMALL_CASE(32, 32, 4, 8, 2)
-    FLINT_SMALL_CASE(32, 64, 4, 6, 2)
-    FLINT_SMALL_CASE(64, 64, 8, 8, 2)
-    FLINT_SMALL_CASE(64, 64, 4, 4, 1)
-    FLINT_SMALL_CASE(128, 64, 8, 3, 1)
+    FLINT_SMALL_CASE(32, 32, 5, 8, 2, true)
+    FLINT_SMALL_CASE(32, 64, 4, 6, 2, false)
+    FLINT_SMALL_CASE(64, 64, 8, 6, 2, true)
+    FLINT_SMALL_CASE(64, 64, 4, 4, 1, false)
+    FLINT_SMALL_CASE(128, 64, 8, 3, 1, false)
 #undef FLINT_SMALL_CASE
     return hipErrorInvalidValue;
 }
@@ -574,6 +575,9 @@ bool gemm_small_plan(GemmLayout l, Epilogue e, size_t slices, size_t m, size_t n
     // (8192 x 50257 x 768 1486 against 1592).
     if (best == kNoEstimate && !force && small_tiles(kSmallConfigs[4], slices, m, n) > 96.0 * cus)
         return false;
+    // Only for a clear gain, so that no product gets slower by an estimate's
+    // error (NN 1500 x 2272 x 568: 11.7 us here, 10.3 in the pipeline).
+    if (best != kNoEstimate) best *= 0.9;
     bool taken = false;
     for (const SmallConfig& c : kSmallConfigs) {
         if (force && (c.bm != forced.bm || c.bn != forced.bn || c.waves != forced.waves)) continue;

@@ -12,7 +12,7 @@ from inputs import normal, uniform
 
 pytestmark = pytest.mark.gpu
 
-CONFIGS = ["32,32,4,8,2", "32,64,4,6,2", "64,64,8,8,2", "64,64,4,4,1", "128,64,8,3,1"]
+CONFIGS = ["32,32,5,8,2", "32,64,4,6,2", "64,64,8,6,2", "64,64,4,4,1", "128,64,8,3,1"]
 H, F = torch.float16, torch.float32
 GUARD = 1024
 
