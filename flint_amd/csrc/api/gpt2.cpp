@@ -134,6 +134,9 @@ struct flint_gpt2 {
     // runs at once).
     size_t ln_offset = 0;
     mutable flint::ParamsMerge pending{};
+    // A layer's bias gradient over few rows that waits for the next one, to
+    // share its launch (within one backward call, while its dy stands).
+    mutable flint::BiasGradient pending_bias{};
     // The attention plan of the last forward, which its backward follows
     // (plan overrides may change in between).
     AttnPlan attn_plan = AttnPlan::kCopies;
@@ -616,17 +619,29 @@ flint_status bias_grad(const flint_gpt2& m, const Param& p, const void* dy, int 
     return flint_bias_gradient(p.grad, dy, m.rows, p.cols, acc, m.work, m.work_bytes, st);
 }
 
+// Runs the bias gradient that waits, with `next` in its launch.
+flint_status flush_bias(const flint_gpt2& m, const flint::BiasGradient& next, flint_stream st) {
+    const flint::BiasGradient first = m.pending_bias.cols > 0 ? m.pending_bias : next;
+    const flint::BiasGradient second = m.pending_bias.cols > 0 ? next : flint::BiasGradient{};
+    m.pending_bias = flint::BiasGradient{};
+    if (first.cols == 0) return FLINT_OK;
+    FLINT_HIP_CHECK(flint::launch_bias_gradients_few(first, second, m.rows, flint::to_hip(st)));
+    return FLINT_OK;
+}
+
 // A linear layer's weight and bias gradients from its output gradient dy
 // (FP16, rows x w.rows) and input x: the TN product into its k-split
 // partials, the bias's chunk partials, then one launch that sums the first
 // and merges the second, in place of flint_gemm_tn's and
 // flint_bias_gradient's two launches each (the same kernels' arithmetic, the
 // same bits). The "fused_grads" override "0" calls the two entry points
-// instead (the tests compare the two).
+// instead (the tests compare the two). `pair`: another layer's linear_grads
+// follows while dy stands, whose launch may then take this bias gradient too.
 flint_status linear_grads(const flint_gpt2& m, const Param& w, const Param& b, const void* dy,
-                          const void* x, int acc, flint_stream st) {
+                          const void* x, int acc, flint_stream st, bool pair = false) {
     const hipStream_t hs = flint::to_hip(st);
     if (flint::tuning_off(flint::Tune::kFusedGrads)) {
+        FLINT_TRY(flush_bias(m, {}, st));
         FLINT_TRY(flush_merge(m, st));
         FLINT_TRY(weight_grad(m, w, dy, x, acc, st));
         return bias_grad(m, b, dy, acc, st);
@@ -642,9 +657,12 @@ flint_status linear_grads(const flint_gpt2& m, const Param& w, const Param& b, c
     // Few rows: the weight gradient unsplit and the bias gradient in a launch
     // of its own leave the finish nothing to do.
     if (splits == 1 && flint::bias_gradient_one_launch(m.rows, b.cols)) {
-        FLINT_HIP_CHECK(flint::launch_bias_gradient(b.grad, dy, m.rows, b.cols, acc != 0, m.work, hs));
+        const flint::BiasGradient bias{b.grad, dy, b.cols, acc != 0};
+        if (pair) m.pending_bias = bias;
+        else FLINT_TRY(flush_bias(m, bias, st));
         return flush_merge(m, st);
     }
+    FLINT_TRY(flush_bias(m, {}, st));
     FLINT_HIP_CHECK(flint::launch_bias_partials(m.work, dy, m.rows, b.cols, hs));
     // The finish also carries a LayerNorm backward's deferred merge.
     FLINT_HIP_CHECK(flint::launch_linear_grads_finish(w.grad, m.tn_work, w.rows, w.cols, splits,
@@ -695,13 +713,14 @@ flint_status backward_layer(const flint_gpt2& m, const Layer& L, int acc, flint_
 
     // dres_half = RN16(dres): written by the LayerNorm backward that produced
     // dres (norm_backward), in place of the reference's conversion here.
-    FLINT_TRY(linear_grads(m, *L.fc_proj.w, *L.fc_proj.b, m.dres_half, s.gelu, acc, st));
+    FLINT_TRY(linear_grads(m, *L.fc_proj.w, *L.fc_proj.b, m.dres_half, s.gelu, acc, st, true));
     FLINT_TRY(flint_gemm_nn_dgelu(m.dpre, m.dres_half, L.fc_proj.half, s.pre, rows, 4 * w, w, st));
     FLINT_TRY(linear_grads(m, *L.fc.w, *L.fc.b, m.dpre, s.h2, acc, st));
     FLINT_TRY(flint_gemm_nn(m.dh, m.dpre, L.fc.half, rows, w, 4 * w, st));
     FLINT_TRY(norm_backward(m, L.ln_2, s.x_mid, s.mean2, s.rstd2, 1, acc, st));
 
-    FLINT_TRY(linear_grads(m, *L.attn_proj.w, *L.attn_proj.b, m.dres_half, s.attn_out, acc, st));
+    FLINT_TRY(linear_grads(m, *L.attn_proj.w, *L.attn_proj.b, m.dres_half, s.attn_out, acc, st,
+                           true));
     FLINT_TRY(flint_gemm_nn(m.dh, m.dres_half, L.attn_proj.half, rows, w, w, st));
     if (m.flash) {
         // dO rows in dh, O in attn_out, q, k, v in the saved projection; dq,
@@ -921,6 +940,7 @@ FLINT_API flint_status flint_gpt2_backward(flint_gpt2* model, const void* tokens
                       "tokens and the gradient of %s overlap", p.name.c_str());
     FLINT_TRY(check.status());
     m.pending = flint::ParamsMerge{};   // nothing carries over from an earlier call
+    m.pending_bias = flint::BiasGradient{};
     // Output layer (tied to wte): dwte (+)= dlogits^T h_f; dh = dlogits wte.
     FLINT_TRY(weight_grad(m, *m.wte, m.dlogits, m.h_f, accumulate, stream));
     FLINT_TRY(flint_gemm_nn(m.dh, m.dlogits, m.wte_half, rows, w, c.padded_vocab, stream));

@@ -207,6 +207,16 @@ hipError_t launch_bias_gradient(void* dbias, const void* dy, size_t rows, size_t
                                 bool accumulate, void* workspace, hipStream_t stream);
 // Whether launch_bias_gradient takes this shape in one launch (no workspace).
 bool bias_gradient_one_launch(size_t rows, size_t cols);
+// Two bias gradients over the same number of rows that each take one launch
+// (bias_gradient_one_launch), in one; an empty one (cols 0) is none.
+struct BiasGradient {
+    void* dbias = nullptr;
+    const void* dy = nullptr;
+    size_t cols = 0;
+    bool accumulate = false;
+};
+hipError_t launch_bias_gradients_few(const BiasGradient& one, const BiasGradient& two, size_t rows,
+                                     hipStream_t stream);
 // The same two passes with the partials in the library's per-device scratch
 // array (kBiasGradientScratchBytes; no allocation). Sizes whose partials do
 // not fit return hipErrorInvalidValue.

@@ -7,8 +7,10 @@ import numpy as np
 import pytest
 import torch
 
+import gpt2_model as G
 from inputs import normal
 from oracle import oracle
+from test_gpt2 import _dev16, _load, _make, _tokens
 
 pytestmark = pytest.mark.gpu
 
@@ -64,3 +66,31 @@ def test_layernorm_parameter_sums(flint, cuda, tune, rows, cols, accumulate):
         assert np.array_equal(_bits(a), _bits(b))
     ref = oracle.bias_gradient(dy.numpy(), normal((cols,), 16).numpy() if accumulate else None)
     assert np.array_equal(_bits(got[2]), _bits(ref))
+
+
+@pytest.mark.parametrize("sequences,length", [(1, 8), (4, 64), (1, 264), (16, 72), (32, 64)])
+def test_model_bias_gradients(flint, cuda, tune, sequences, length):
+    """Two layers' bias gradients in one launch (widths 96 beside 384, 288
+    beside 96: a part of a column block at either end) against two passes each,
+    in a fresh and in an accumulating backward."""
+    cfg = dict(layers=2, heads=3, width=96, block_size=272, vocab=997, padded_vocab=1000)
+    shapes = G.parameter_shapes(cfg["layers"], cfg["width"], cfg["block_size"],
+                                cfg["padded_vocab"])
+    params = G.init_params(shapes, cfg["layers"], cfg["vocab"], seed=3, trained=True)
+    idx, tgt = _tokens(cfg, sequences, length, 4)
+
+    def run():
+        with _make(flint, cfg, sequences, length) as model:
+            _load(model, params)
+            tok = _dev16(idx)
+            model.forward(tok, _dev16(tgt), 0.5)
+            model.backward(tok)
+            model.backward(tok, accumulate=True)
+            torch.cuda.synchronize()
+            return {n: model.read(a, (r, c), torch.float32).cpu() for n, a, r, c in model.gradients()
+                    if n.endswith("bias")}
+
+    got = run()
+    tune("sums_few", "0")
+    for n, g in run().items():
+        assert torch.equal(g.view(torch.int32), got[n].view(torch.int32)), n
