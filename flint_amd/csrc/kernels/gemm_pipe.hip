@@ -1,7 +1,8 @@
 // The GEMM pipeline on gfx950 with one wave per SIMD and large wave tiles,
-// for all three layouts (NT, NN, TN, and their batched forms) whenever k is a
-// multiple of 32 and the output rows are 16-byte multiples. Products of few
-// tiles run gemm_small.hip's kernels, other shapes gemm.hip's.
+// for all three layouts (NT, NN, TN, and their batched forms) where rows of
+// operands and output are 16-byte multiples (TN's FP32 output: any k; batched
+// products: k a multiple of 32). Products of few tiles and most ragged ones
+// run gemm_small.hip's kernels, what is left gemm.hip's.
 //
 // Why this shape of kernel (measured on MI355X):
 //  * A CU's L2 -> LDS rate depends on the row piece one load covers: 64-byte

@@ -143,6 +143,8 @@ __global__ void __launch_bounds__(NW * 64) gemm_small(Operands op, TileArgs ta) 
     // ---- operand loads. Row-major: a resource over the tile's valid rows,
     // the k-step in the scalar offset, chunks past k_end sent outside.
     // k-major: a resource from the step's first k row to the operand's end.
+    // Offsets within a tile fit in 32 bits: the entry points take k up to 65,536
+    // (kGemmMaxK) and m and n up to 8,388,480 (kGemmMaxMN).
     const _Float16* const a = kXM ? xs + m0 : xs + size_t(m0) * K;
     const _Float16* const b = kWM ? ws + n0 : ws + size_t(n0) * K;
     const size_t a_bytes = kXM ? (size_t(K) * m - m0) * 2 : size_t(min(BM, m - m0)) * K * 2;

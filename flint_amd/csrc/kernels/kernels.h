@@ -176,8 +176,9 @@ constexpr size_t layernorm_backward_workspace(size_t rows, size_t cols) {
 hipError_t launch_layernorm_forward(void* y, void* mean, void* rstd, const void* x,
                                     const void* gamma, const void* beta, size_t rows, size_t cols,
                                     float eps, hipStream_t stream);
-// LayerNorm backward in two launches: the dbeta and dgamma chunk partials from
-// one pass over dy and x, then dx, whose kernel also merges the partials.
+// LayerNorm backward: dx and the dbeta and dgamma chunk partials from one pass
+// over dy and x, then a merge of the partials (rows of one chunk merge in the
+// first launch).
 // With dx_half, RN16 of every dx value written goes there too (the values
 // flint_fp32_to_fp16 of dx would give). workspace:
 // layernorm_backward_workspace(rows, cols) bytes.
