@@ -960,7 +960,7 @@ hipError_t launch_gemm_nn_batched_views(void* y, const void* x, const void* w, s
                                         const HeadView& yv, hipStream_t stream, bool causal) {
     if (!gemm_pipe_eligible(GemmLayout::kNN, Epilogue::kNone, m, n, k)) return hipErrorInvalidValue;
     SmallPlan small;
-    if (gemm_small_plan(GemmLayout::kNN, Epilogue::kNone, batches, m, n, k, 1, &small))
+    if (gemm_small_plan(GemmLayout::kNN, Epilogue::kNone, batches, m, n, k, 1, &small, true))
         return launch_gemm_small(small, GemmLayout::kNN, Epilogue::kNone, y, x, w, nullptr, nullptr,
                                  1.0f, batches, m, n, k, false, nullptr, stream,
                                  causal && m == k, &wv, &yv);
@@ -974,7 +974,7 @@ hipError_t launch_gemm_tn_batched_views(void* y, const void* x, const void* w, s
                                         const HeadView& yv, hipStream_t stream, bool causal) {
     if (!gemm_pipe_eligible(GemmLayout::kTN, Epilogue::kNone, m, n, k)) return hipErrorInvalidValue;
     SmallPlan small;
-    if (gemm_small_plan(GemmLayout::kTN, Epilogue::kNone, batches, m, n, k, 1, &small))
+    if (gemm_small_plan(GemmLayout::kTN, Epilogue::kNone, batches, m, n, k, 1, &small, true))
         return launch_gemm_small(small, GemmLayout::kTN, Epilogue::kNone, y, x, w, nullptr, nullptr,
                                  1.0f, batches, m, n, k, false, nullptr, stream,
                                  causal && m == k, &wv, &yv);

@@ -997,11 +997,12 @@ size_t lds_bytes(const PipeConfig& c, Store st) {
 bool has_tail(const PipeConfig& c) { return c.same(PipeConfig{128, 192, 3, 64}); }
 
 // Whether a configuration can run an epilogue over k: it fits in LDS and k is
-// whole k-steps, or TN's FP32 output's, or the configuration takes tails; the 8-wave
-// configuration serves the NT layout only.
-bool usable(const PipeConfig& c, Store st, size_t k, Layout l) {
-    return lds_bytes(c, st) <= kPipeMaxLds &&
-           (k % size_t(c.bk) == 0 || st == Store::kTn || (l != Layout::kTN && has_tail(c))) &&
+// whole k-steps, or TN's FP32 output's, or the configuration takes tails (its
+// heads-view instances do not); the 8-wave configuration serves the NT layout
+// only.
+bool usable(const PipeConfig& c, Store st, size_t k, Layout l, bool views) {
+    const bool tail = st == Store::kTn || (l != Layout::kTN && !views && has_tail(c));
+    return lds_bytes(c, st) <= kPipeMaxLds && (k % size_t(c.bk) == 0 || tail) &&
            (c.waves == 4 || l == Layout::kNT);
 }
 
@@ -1063,11 +1064,11 @@ double pipe_eff(const PipeConfig& c, Store st, Layout l) {
 constexpr double kPipe8MinRounds = 8.0;
 
 PipeConfig pick_pipe(size_t m, size_t n, size_t k, size_t slices, int cus, Store st, Layout l,
-                     bool causal = false) {
+                     bool views, bool causal = false) {
     PipeConfig best = kPipeConfigs[0];
     double best_cost = 1e300;
     for (const PipeConfig& c : kPipeConfigs) {
-        if (!usable(c, st, k, l)) continue;
+        if (!usable(c, st, k, l, views)) continue;
         // 64-wide tiles only for outputs that narrow: elsewhere a round of
         // them costs as much as one of the wider tiles and loads far more.
         if (c.bn == 64 && n > 64) continue;
@@ -1105,10 +1106,10 @@ void plan_tn(size_t m, size_t n, size_t k, int max_splits, int cus, bool accumul
              const PipeConfig* only, PipeConfig* best_c, int* best_s) {
     const Store st = Store::kTn;
     double best = 1e300;
-    *best_c = only != nullptr ? *only : pick_pipe(m, n, k, 1, cus, st, Layout::kTN);
+    *best_c = only != nullptr ? *only : pick_pipe(m, n, k, 1, cus, st, Layout::kTN, false);
     *best_s = 1;
     for (const PipeConfig& c : kPipeConfigs) {
-        if (!usable(c, st, k, Layout::kTN)) continue;
+        if (!usable(c, st, k, Layout::kTN, false)) continue;
         if (only != nullptr && !c.same(*only)) continue;
         if (only == nullptr && c.bn == 64 && (n > 64 || c.bm == 128)) continue;
         // The 256 x 128 loader tile won only on the logits' size of output.
@@ -1160,9 +1161,13 @@ hipError_t launch_pipe(const PipeConfig& c, const Operands& op, size_t slices, i
     size_t gx = std::min(total, size_t(cus));
     if (gx >= 8) gx -= gx % 8;
     const dim3 grid(unsigned(gx), 1, 1);
+    // Only the k-tail instances and TN's FP32 output have a partial last k-step:
+    // any other would drop the k past the whole ones.
+    const bool whole = ST == Store::kTn || op.k % c.bk == 0;
 #define FLINT_PIPE_CASE(BM_, BN_, S_, BK_, NW_, LD_)                                           \
     if constexpr (pipe_lds_bytes<BM_, BN_, S_, BK_, L, ST, NW_>() <= kPipeMaxLds) {            \
         if (c.same(PipeConfig{BM_, BN_, S_, BK_, NW_, LD_})) {                                 \
+            if (hv && !whole) return hipErrorInvalidValue;                                     \
             if constexpr (kViews) {                                                            \
                 if (hv) {                                                                      \
                     hipLaunchKernelGGL((gemm_pipe<BM_, BN_, S_, BK_, L, ST, NW_, LD_ != 0,     \
@@ -1173,13 +1178,14 @@ hipError_t launch_pipe(const PipeConfig& c, const Operands& op, size_t slices, i
             }                                                                                  \
             if (hv) return hipErrorInvalidValue;                                               \
             if constexpr (L != Layout::kTN && BM_ == 128 && BN_ == 192 && BK_ == 64 && LD_ == 0) { \
-                if (op.k % BK_ != 0) {                                                         \
+                if (!whole) {                                                                  \
                     hipLaunchKernelGGL((gemm_pipe<BM_, BN_, S_, BK_, L, ST, NW_, false, false, \
                                                   true>),                                      \
                                        grid, dim3(NW_ * 64), 0, stream, op, ta);               \
                     return hipGetLastError();                                                  \
                 }                                                                              \
             }                                                                                  \
+            if (!whole) return hipErrorInvalidValue;                                           \
             hipLaunchKernelGGL((gemm_pipe<BM_, BN_, S_, BK_, L, ST, NW_, LD_ != 0>), grid,     \
                                dim3((NW_ + 4 * LD_) * 64), 0, stream, op, ta);                 \
             return hipGetLastError();                                                          \
@@ -1266,7 +1272,7 @@ hipError_t launch_gemm_pipe_tn(void* y, const void* x, const void* w, size_t m, 
     int sp = 1;
     bool disabled = false;
     PipeConfig forced;
-    const bool force = pipe_forced(&forced, &disabled) && usable(forced, Store::kTn, k, Layout::kTN);
+    const bool force = pipe_forced(&forced, &disabled) && usable(forced, Store::kTn, k, Layout::kTN, false);
     plan_tn(m, n, k, workspace != nullptr ? max_splits : 1, cus, accumulate,
             force ? &forced : nullptr, &c, &sp);
     const size_t len = ((k + sp - 1) / sp + c.bk - 1) / c.bk * c.bk;
@@ -1321,7 +1327,7 @@ bool gemm_pipe_eligible(GemmLayout gl, Epilogue e, size_t m, size_t n, size_t k)
 // take 2.7 to 2.8 us, TN's FP32 output 4.6. The constants are fitted together with
 // gemm_small.hip's.
 double gemm_pipe_estimate(GemmLayout gl, Epilogue e, size_t slices, size_t m, size_t n, size_t k,
-                          int max_splits) {
+                          int max_splits, bool views) {
     constexpr double kInfinite = 1e300;
     int cus = 256;
     if (!gemm_pipe_eligible(gl, e, m, n, k) || device_cus(&cus) != hipSuccess) return kInfinite;
@@ -1330,7 +1336,7 @@ double gemm_pipe_estimate(GemmLayout gl, Epilogue e, size_t slices, size_t m, si
     PipeConfig c;
     int sp = 1;
     if (e == kTnFloat) plan_tn(m, n, k, max_splits, cus, false, nullptr, &c, &sp);
-    else c = pick_pipe(m, n, k, slices, cus, st, l);
+    else c = pick_pipe(m, n, k, slices, cus, st, l, views);
     const double tiles = double((m + c.bm - 1) / c.bm) * double((n + c.bn - 1) / c.bn) *
                          double(slices) * sp;
     const double rounds = std::ceil(tiles / cus);
@@ -1402,8 +1408,9 @@ hipError_t launch_gemm_pipe(GemmLayout gl, Epilogue e, void* y, const void* x, c
     const Store st = store_of(e, l);
     PipeConfig c;
     bool disabled = false;
-    if (!pipe_forced(&c, &disabled) || !usable(c, st, k, l))
-        c = pick_pipe(m, n, k, slices, cus, st, l, op.causal != 0);
+    const bool views = op.wv.heads != 0;
+    if (!pipe_forced(&c, &disabled) || !usable(c, st, k, l, views))
+        c = pick_pipe(m, n, k, slices, cus, st, l, views, op.causal != 0);
     switch (l) {
     case Layout::kNT: return dispatch_pipe<Layout::kNT>(c, st, op, slices, split_len, cus, stream);
     case Layout::kNN: return dispatch_pipe<Layout::kNN>(c, st, op, slices, split_len, cus, stream);

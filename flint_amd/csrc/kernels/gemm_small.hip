@@ -561,7 +561,7 @@ hipError_t launch(const SmallPlan& c, const Operands& op, size_t slices, hipStre
 // not take the shape). Either side gives the same sums, so the line only has
 // to be about right.
 bool gemm_small_plan(GemmLayout l, Epilogue e, size_t slices, size_t m, size_t n, size_t k,
-                     int max_splits, SmallPlan* plan) {
+                     int max_splits, SmallPlan* plan, bool views) {
     SmallConfig forced;
     bool disabled = false;
     const bool force = small_forced(&forced, &disabled);
@@ -570,7 +570,7 @@ bool gemm_small_plan(GemmLayout l, Epilogue e, size_t slices, size_t m, size_t n
     if (!force && tuning(Tune::kGemmPipe) != nullptr) return false;
     int cus = 256;
     if (device_cus(&cus) != hipSuccess) return false;
-    double best = force ? kNoEstimate : gemm_pipe_estimate(l, e, slices, m, n, k, max_splits);
+    double best = force ? kNoEstimate : gemm_pipe_estimate(l, e, slices, m, n, k, max_splits, views);
     // Ragged products the pipeline does not take would run gemm.hip's kernels:
     // slower up to about 60 rounds of 128 x 64 tiles (NT 2500 x 50257 x 768 465
     // against 446 us here; 6753 x 800 x 200 14.9 against 11.2), faster at 196

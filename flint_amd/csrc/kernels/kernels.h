@@ -49,9 +49,9 @@ hipError_t launch_gemm_pipe(GemmLayout l, Epilogue e, void* y, const void* x, co
                             const HeadView* wv = nullptr, const HeadView* yv = nullptr);
 // The pipeline's estimated time for a product, us past a launch's own, with
 // the tile (and TN split, up to max_splits) it would choose; infinite where it
-// does not take the shape.
+// does not take the shape. views: the product reads and writes heads views.
 double gemm_pipe_estimate(GemmLayout l, Epilogue e, size_t slices, size_t m, size_t n, size_t k,
-                          int max_splits);
+                          int max_splits, bool views);
 // GEMMs of few tiles (gemm_small.hip), every layout, epilogue and size: the
 // launchers below run there where gemm_small_plan says so. max_splits: TN's
 // FP32 output may split k up to that often (the count is plan->splits, the
@@ -62,7 +62,7 @@ struct SmallPlan {
     int splits, split_len;
 };
 bool gemm_small_plan(GemmLayout l, Epilogue e, size_t slices, size_t m, size_t n, size_t k,
-                     int max_splits, SmallPlan* plan);
+                     int max_splits, SmallPlan* plan, bool views = false);
 hipError_t launch_gemm_small(const SmallPlan& plan, GemmLayout l, Epilogue e, void* y, const void* x,
                              const void* w, const void* bias, void* aux, float scale,
                              size_t slices, size_t m, size_t n, size_t k, bool accumulate,

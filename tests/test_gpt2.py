@@ -325,7 +325,8 @@ def test_fused_scores_and_softmax_change_no_bits(flint, cuda, tune, length, caus
 
 @pytest.mark.parametrize("length", [1024, 320, 96, 32])
 @pytest.mark.parametrize("causal", ["1", "0"], ids=["causal", "full"])
-def test_head_views_change_no_bits(flint, cuda, tune, length, causal):
+@pytest.mark.parametrize("small", [None, "0"], ids=["default", "pipeline"])
+def test_head_views_change_no_bits(flint, cuda, tune, length, causal, small):
     """In one allocation the stored-probability model reads q, k, v and dO and
     writes O, dQ, dK and dV as heads views of the token rows, with no split or
     merge copies; separate buffers (q, k, v not back to back) run the copies
@@ -340,6 +341,8 @@ def test_head_views_change_no_bits(flint, cuda, tune, length, causal):
     idx, tgt = _tokens(cfg, sequences, length, 18)
     if causal == "0":
         tune("attn_causal", "0")
+    if small is not None:
+        tune("gemm_small", small)
     views = _run(flint, cfg, sequences, length, params, idx, tgt, 0.25)
     copies = _run(flint, cfg, sequences, length, params, idx, tgt, 0.25, separate=True)
     for x, y in zip(copies[:3], views[:3]):
@@ -349,6 +352,38 @@ def test_head_views_change_no_bits(flint, cuda, tune, length, causal):
         assert torch.equal(copies[3][n].view(torch.int32), views[3][n].view(torch.int32)), n
     assert copies[4] == views[4]
     assert bool(torch.isfinite(views[1]).all())
+
+
+@pytest.mark.parametrize("length", [32, 96, 160])
+@pytest.mark.parametrize("causal", ["1", "0"], ids=["causal", "full"])
+@pytest.mark.parametrize("plan", [dict(gemm_small="0"),
+                                  dict(gemm_small="0", gemm_pipe="128,192,3,64"),
+                                  dict(gemm_small="0", gemm_pipe="128,64,3,64")],
+                         ids=["pipeline", "tail-tile", "64-deep"])
+def test_pipeline_head_views_take_every_key(flint, cuda, tune, length, causal, plan):
+    """Lengths that are not whole 64-deep k-steps: P V and dS K over heads
+    views must sum every key whichever pipeline tile is asked for, also the
+    one whose plain instances take a partial last step (its views do not). The
+    few-tile kernels, in one chain over the same keys, give the bits."""
+    cfg = dict(layers=1, heads=3, width=192, block_size=1024, vocab=1000, padded_vocab=1024)
+    sequences = 2
+    shapes = G.parameter_shapes(cfg["layers"], cfg["width"], cfg["block_size"],
+                                cfg["padded_vocab"])
+    params = G.init_params(shapes, cfg["layers"], cfg["vocab"], seed=19, trained=True)
+    params = {n: t.half().float() for n, t in params.items()}
+    idx, tgt = _tokens(cfg, sequences, length, 20)
+    if causal == "0":
+        tune("attn_causal", "0")
+    with flint.tuned(gemm_small="64,64,4,4,1"):
+        ref = _run(flint, cfg, sequences, length, params, idx, tgt, 0.25)
+    with flint.tuned(**plan):
+        got = _run(flint, cfg, sequences, length, params, idx, tgt, 0.25)
+    for x, y in zip(ref[:3], got[:3]):
+        assert torch.equal(x.view(torch.int32) if x.dtype == torch.float32 else x,
+                           y.view(torch.int32) if y.dtype == torch.float32 else y)
+    for n in ref[3]:
+        assert torch.equal(ref[3][n].view(torch.int32), got[3][n].view(torch.int32)), n
+    assert ref[4] == got[4]
 
 
 WIDE = dict(layers=1, heads=4, width=256, block_size=1024, vocab=1000, padded_vocab=1024)
