@@ -499,6 +499,9 @@ double small_cost(const SmallConfig& c, GemmLayout l, double tiles, double steps
            steps * std::max(c.alone[i], full * c.shared[i]);
 }
 
+// A launch holds fewer than 2^32 threads along x.
+bool fits_a_launch(double tiles, int waves) { return tiles * waves * 64 <= double(0xffffffffu); }
+
 double small_tiles(const SmallConfig& c, size_t slices, size_t m, size_t n) {
     return double((m + c.bm - 1) / c.bm) * double((n + c.bn - 1) / c.bn) * double(slices);
 }
@@ -532,7 +535,7 @@ hipError_t launch(const SmallPlan& c, const Operands& op, size_t slices, hipStre
     ta.tiles_m = (op.m + c.bm - 1) / c.bm;
     ta.tiles_n = (op.n + c.bn - 1) / c.bn;
     const size_t per = size_t(ta.tiles_m) * size_t(ta.tiles_n);
-    if (per * slices > 0x7fffffffu) return hipErrorInvalidValue;
+    if (!fits_a_launch(double(per) * double(slices), c.waves)) return hipErrorInvalidValue;
     ta.tiles_per_slice = int(per);
     ta.slices = int(slices);
     ta.group_m = 8;
@@ -584,10 +587,10 @@ bool gemm_small_plan(GemmLayout l, Epilogue e, size_t slices, size_t m, size_t n
     for (const SmallConfig& c : kSmallConfigs) {
         if (force && (c.bm != forced.bm || c.bn != forced.bn || c.waves != forced.waves)) continue;
         const double tiles = small_tiles(c, slices, m, n);
-        if (tiles > double(0x7fffffff)) continue;
+        if (!fits_a_launch(tiles, c.waves)) continue;
         for (int sp = 1; sp <= max_splits; ++sp) {
             const size_t len = ((k + sp - 1) / sp + kStep - 1) / kStep * kStep;
-            if (size_t(sp - 1) * len >= k || tiles * sp > double(0x7fffffff)) break;
+            if (size_t(sp - 1) * len >= k || !fits_a_launch(tiles * sp, c.waves)) break;
             double cost = small_cost(c, l, tiles * sp, double(len / kStep), cus);
             if (sp > 1) cost += kSplitSumUs + double(sp + 2) * double(m) * double(n) * 4.0 / 5e6;
             if (cost < best) {

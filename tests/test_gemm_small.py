@@ -180,3 +180,19 @@ def test_pipeline_tn_takes_any_k(flint, cuda, cfg, m, n, k):
     ref = x.double().t() @ w.double()
     bound = 2 * k * 2.0 ** -24 * (x.double().abs().t() @ w.double().abs()) + 2.0 ** -22 * ref.abs()
     assert bool(((got.double() - ref).abs() <= bound).all())
+
+
+def test_more_tiles_than_a_launch_holds(flint, cuda):
+    """13.6 million 32 x 32 tiles of 320 threads are past the 2^32 threads of a
+    launch: the forced configuration cannot run and the product runs as it
+    would have, every value right (small whole numbers, exact in FP16)."""
+    m, n, k = 8388480, 1664, 8
+    x = (uniform((m, k), 41) * 4).round().to(cuda)
+    w = (uniform((n, k), 42) * 4).round().to(cuda)
+    y = torch.full((m, n), float("nan"), dtype=H, device=cuda)
+    with flint.tuned(gemm_small="32,32,5,8,2"):
+        flint.gemm_nt(y, x, w, m, n, k)
+    torch.cuda.synchronize()
+    wt = w.float().t().contiguous()
+    for r in range(0, m, 262140):
+        assert torch.equal(y[r:r + 262140].float(), x[r:r + 262140].float() @ wt), r
