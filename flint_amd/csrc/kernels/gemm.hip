@@ -789,6 +789,20 @@ Operands make_ops(void* y, const void* x, const void* w, size_t m, size_t n, siz
     return op;
 }
 
+// Which kernels run a product. A "gemm_config" override keeps here what the
+// pipeline does not take in whole 32-deep steps, unless "gemm_small" names a
+// few-tile configuration.
+enum class Route { kFewTiles, kPipeline, kHere };
+Route route(GemmLayout l, Epilogue e, size_t slices, size_t m, size_t n, size_t k, int max_splits,
+            SmallPlan* small) {
+    const bool pipe = gemm_pipe_eligible(l, e, m, n, k);
+    Config forced;
+    if (forced_config(&forced) && !(pipe && k % 32 == 0) && !gemm_small_override())
+        return Route::kHere;
+    if (gemm_small_plan(l, e, slices, m, n, k, max_splits, small)) return Route::kFewTiles;
+    return pipe ? Route::kPipeline : Route::kHere;
+}
+
 // TN's split of k. The count is the smallest that keeps at least 3/4 of the
 // CUs busy over all waves of tiles (or the fullest, up to 16 splits), each split
 // at least 1,024 long and a multiple of 64; the last split takes the rest.
@@ -836,10 +850,11 @@ hipError_t gemm_tn_workspace(size_t m, size_t n, size_t k, size_t* bytes) {
 hipError_t launch_gemm_nt(void* y, const void* x, const void* w, const void* bias, void* aux,
                           Epilogue e, size_t m, size_t n, size_t k, hipStream_t stream) {
     SmallPlan small;
-    if (gemm_small_plan(GemmLayout::kNT, e, 1, m, n, k, 1, &small))
+    const Route to = route(GemmLayout::kNT, e, 1, m, n, k, 1, &small);
+    if (to == Route::kFewTiles)
         return launch_gemm_small(small, GemmLayout::kNT, e, y, x, w, bias, aux, 1.0f, 1, m, n, k,
                                  false, nullptr, stream);
-    if (gemm_pipe_eligible(GemmLayout::kNT, e, m, n, k))
+    if (to == Route::kPipeline)
         return launch_gemm_pipe(GemmLayout::kNT, e, y, x, w, bias, aux, 1.0f, 1, m, n, k, false,
                                 nullptr, 0, stream);
     Operands op = make_ops(y, x, w, m, n, k);
@@ -857,10 +872,11 @@ hipError_t launch_gemm_nt(void* y, const void* x, const void* w, const void* bia
 hipError_t launch_gemm_nn(void* y, const void* x, const void* w, const void* aux, Epilogue e,
                           size_t m, size_t n, size_t k, hipStream_t stream) {
     SmallPlan small;
-    if (gemm_small_plan(GemmLayout::kNN, e, 1, m, n, k, 1, &small))
+    const Route to = route(GemmLayout::kNN, e, 1, m, n, k, 1, &small);
+    if (to == Route::kFewTiles)
         return launch_gemm_small(small, GemmLayout::kNN, e, y, x, w, nullptr, const_cast<void*>(aux),
                                  1.0f, 1, m, n, k, false, nullptr, stream);
-    if (gemm_pipe_eligible(GemmLayout::kNN, e, m, n, k))
+    if (to == Route::kPipeline)
         return launch_gemm_pipe(GemmLayout::kNN, e, y, x, w, nullptr, const_cast<void*>(aux), 1.0f,
                                 1, m, n, k, false, nullptr, 0, stream);
     Operands op = make_ops(y, x, w, m, n, k);
@@ -882,13 +898,14 @@ hipError_t launch_gemm_tn_split(void* y, const void* x, const void* w, size_t m,
     op.partials = splits > 1 ? static_cast<float*>(workspace) : nullptr;
     hipError_t err;
     SmallPlan small;
-    if (gemm_small_plan(GemmLayout::kTN, kTnFloat, 1, m, n, k, op.partials != nullptr ? splits : 1,
-                        &small)) {
+    const Route to = route(GemmLayout::kTN, kTnFloat, 1, m, n, k,
+                           op.partials != nullptr ? splits : 1, &small);
+    if (to == Route::kFewTiles) {
         // Its own split count, at most the plan's, like the pipeline.
         splits = small.splits;
         err = launch_gemm_small(small, GemmLayout::kTN, kTnFloat, y, x, w, nullptr, nullptr, 1.0f, 1,
                                 m, n, k, accumulate, splits > 1 ? op.partials : nullptr, stream);
-    } else if (gemm_pipe_eligible(GemmLayout::kTN, kTnFloat, m, n, k)) {
+    } else if (to == Route::kPipeline) {
         // The pipeline picks its own split count, at most the plan's.
         int used = 1;
         err = launch_gemm_pipe_tn(y, x, w, m, n, k, accumulate, op.partials, splits, &used, stream);
@@ -924,11 +941,12 @@ hipError_t launch_gemm_nt_batched(void* y, const void* x, const void* w, size_t 
                                   size_t m, size_t n, size_t k, float scale, hipStream_t stream,
                                   bool causal) {
     SmallPlan small;
-    if (gemm_small_plan(GemmLayout::kNT, Epilogue::kScale, batches, m, n, k, 1, &small))
+    const Route to = route(GemmLayout::kNT, Epilogue::kScale, batches, m, n, k, 1, &small);
+    if (to == Route::kFewTiles)
         return launch_gemm_small(small, GemmLayout::kNT, Epilogue::kScale, y, x, w, nullptr, nullptr,
                                  scale, batches, m, n, k, false, nullptr, stream,
                                  causal && m == n);
-    if (gemm_pipe_eligible(GemmLayout::kNT, Epilogue::kScale, m, n, k))
+    if (to == Route::kPipeline)
         return launch_gemm_pipe(GemmLayout::kNT, Epilogue::kScale, y, x, w, nullptr, nullptr, scale,
                                 batches, m, n, k, false, nullptr, 0, stream, causal && m == n);
     Operands op = make_ops(y, x, w, m, n, k);
@@ -944,11 +962,12 @@ bool gemm_batched_causal_taken(GemmLayout l, size_t m, size_t n, size_t k) {
 hipError_t launch_gemm_nn_batched(void* y, const void* x, const void* w, size_t batches,
                                   size_t m, size_t n, size_t k, hipStream_t stream, bool causal) {
     SmallPlan small;
-    if (gemm_small_plan(GemmLayout::kNN, Epilogue::kNone, batches, m, n, k, 1, &small))
+    const Route to = route(GemmLayout::kNN, Epilogue::kNone, batches, m, n, k, 1, &small);
+    if (to == Route::kFewTiles)
         return launch_gemm_small(small, GemmLayout::kNN, Epilogue::kNone, y, x, w, nullptr, nullptr,
                                  1.0f, batches, m, n, k, false, nullptr, stream,
                                  causal && m == k);
-    if (gemm_pipe_eligible(GemmLayout::kNN, Epilogue::kNone, m, n, k))
+    if (to == Route::kPipeline)
         return launch_gemm_pipe(GemmLayout::kNN, Epilogue::kNone, y, x, w, nullptr, nullptr, 1.0f,
                                 batches, m, n, k, false, nullptr, 0, stream, causal && m == k);
     Operands op = make_ops(y, x, w, m, n, k);
@@ -986,11 +1005,12 @@ hipError_t launch_gemm_tn_batched_views(void* y, const void* x, const void* w, s
 hipError_t launch_gemm_tn_batched(void* y, const void* x, const void* w, size_t batches,
                                   size_t m, size_t n, size_t k, hipStream_t stream, bool causal) {
     SmallPlan small;
-    if (gemm_small_plan(GemmLayout::kTN, Epilogue::kNone, batches, m, n, k, 1, &small))
+    const Route to = route(GemmLayout::kTN, Epilogue::kNone, batches, m, n, k, 1, &small);
+    if (to == Route::kFewTiles)
         return launch_gemm_small(small, GemmLayout::kTN, Epilogue::kNone, y, x, w, nullptr, nullptr,
                                  1.0f, batches, m, n, k, false, nullptr, stream,
                                  causal && m == k);
-    if (gemm_pipe_eligible(GemmLayout::kTN, Epilogue::kNone, m, n, k))
+    if (to == Route::kPipeline)
         return launch_gemm_pipe(GemmLayout::kTN, Epilogue::kNone, y, x, w, nullptr, nullptr, 1.0f,
                                 batches, m, n, k, false, nullptr, 0, stream, causal && m == k);
     Operands op = make_ops(y, x, w, m, n, k);

@@ -1320,6 +1320,15 @@ bool gemm_pipe_eligible(GemmLayout gl, Epilogue e, size_t m, size_t n, size_t k)
     return true;
 }
 
+bool gemm_pipe_override(GemmLayout gl, Epilogue e, size_t m, size_t n, size_t k, bool views) {
+    bool disabled = false;
+    PipeConfig forced;
+    const bool force = pipe_forced(&forced, &disabled);
+    const Layout l = layout_of(gl);
+    return disabled || (force && gemm_pipe_eligible(gl, e, m, n, k) &&
+                        usable(forced, store_of(e, l), k, l, views));
+}
+
 // Per k-step of 64 a tile takes about 1 us * area / 256^2 / pipe_eff, more
 // where the rounds fill the GPU (the CUs then share the L2s and the power) and
 // where operand rows lie off the 128-byte lines, or are loaded half a line at

@@ -569,8 +569,8 @@ bool gemm_small_plan(GemmLayout l, Epilogue e, size_t slices, size_t m, size_t n
     bool disabled = false;
     const bool force = small_forced(&forced, &disabled);
     if (disabled || m == 0 || n == 0 || k == 0) return false;
-    // A forced pipeline tile means the pipeline.
-    if (!force && tuning(Tune::kGemmPipe) != nullptr) return false;
+    // A forced pipeline tile means the pipeline, and no pipeline gemm.hip.
+    if (!force && gemm_pipe_override(l, e, m, n, k, views)) return false;
     int cus = 256;
     if (device_cus(&cus) != hipSuccess) return false;
     double best = force ? kNoEstimate : gemm_pipe_estimate(l, e, slices, m, n, k, max_splits, views);
@@ -601,6 +601,12 @@ bool gemm_small_plan(GemmLayout l, Epilogue e, size_t slices, size_t m, size_t n
         }
     }
     return taken;
+}
+
+bool gemm_small_override() {
+    SmallConfig forced;
+    bool disabled = false;
+    return small_forced(&forced, &disabled);
 }
 
 hipError_t launch_gemm_small(const SmallPlan& c, GemmLayout l, Epilogue e, void* y, const void* x,

@@ -52,6 +52,9 @@ hipError_t launch_gemm_pipe(GemmLayout l, Epilogue e, void* y, const void* x, co
 // does not take the shape. views: the product reads and writes heads views.
 double gemm_pipe_estimate(GemmLayout l, Epilogue e, size_t slices, size_t m, size_t n, size_t k,
                           int max_splits, bool views);
+// Whether the "gemm_pipe" override decides a product's kernel: it turns the
+// pipeline off, or names a tile that can run the product there.
+bool gemm_pipe_override(GemmLayout l, Epilogue e, size_t m, size_t n, size_t k, bool views);
 // GEMMs of few tiles (gemm_small.hip), every layout, epilogue and size: the
 // launchers below run there where gemm_small_plan says so. max_splits: TN's
 // FP32 output may split k up to that often (the count is plan->splits, the
@@ -63,6 +66,8 @@ struct SmallPlan {
 };
 bool gemm_small_plan(GemmLayout l, Epilogue e, size_t slices, size_t m, size_t n, size_t k,
                      int max_splits, SmallPlan* plan, bool views = false);
+// Whether the "gemm_small" override names a configuration.
+bool gemm_small_override();
 hipError_t launch_gemm_small(const SmallPlan& plan, GemmLayout l, Epilogue e, void* y, const void* x,
                              const void* w, const void* bias, void* aux, float scale,
                              size_t slices, size_t m, size_t n, size_t k, bool accumulate,

@@ -8,10 +8,12 @@
  * set, every entry point runs its default plan.
  *
  * Names and values:
- *   "gemm_pipe"     "0" (no pipeline kernel) or "bm,bn,stages[,bk[,waves[,loaders]]]"
- *   "gemm_small"    "0" (no few-tile kernel) or "bm,bn,waves,stages,unit"
- *   "gemm_config"   "bm,bn,bk,stages,waves_m[,waves]" (the non-pipeline kernel)
- *   "gemm_group_m", "gemm_slots"   positive integers (the non-pipeline kernel)
+ *   "gemm_small"    "0" (no few-tile kernel) or "bm,bn,waves,stages,unit", for every product
+ *   "gemm_pipe"     "0" (no pipeline, and no few-tile kernel unless "gemm_small" names one) or
+ *                   "bm,bn,stages[,bk[,waves[,loaders]]]", for the products this tile can run
+ *   "gemm_config"   "bm,bn,bk,stages,waves_m[,waves]" (the general kernel), for the products the
+ *                   pipeline does not take in whole 32-deep steps of k (with "gemm_pipe" "0": all)
+ *   "gemm_group_m", "gemm_slots"   positive integers (the general kernel)
  *   "attn_causal", "fused_grads", "fused_sums", "ln_defer", "ln_fused",
  *   "emb_together", "attn_order", "attn_scores", "emb_scan", "sums_few"   "0" selects the
  *                   alternative plan

@@ -196,3 +196,30 @@ def test_more_tiles_than_a_launch_holds(flint, cuda):
     wt = w.float().t().contiguous()
     for r in range(0, m, 262140):
         assert torch.equal(y[r:r + 262140].float(), x[r:r + 262140].float() @ wt), r
+
+
+def test_which_overrides_decide_the_kernel(flint, cuda):
+    """TN 768 x 768 x 3000 shows its plan in its bits: by default the few-tile
+    kernels sum k in one piece, the pipeline and the general kernel in two of
+    1,536 and 1,464. A gemm_pipe value that names no tile, or one that cannot
+    run TN, leaves the default; gemm_config, as k is not whole 32-deep steps,
+    means the general kernel."""
+    m, n, k = 768, 768, 3000
+    x = normal((k, m), 43, 0.1, H).to(cuda)
+    w = uniform((k, n), 44).to(cuda)
+    ws = torch.empty(flint.gemm_tn_workspace(m, n, k), dtype=torch.uint8, device=cuda)
+
+    def bits(**plan):
+        got, = _run(flint, lambda y: flint.gemm_tn(y, x, w, m, n, k, workspace=ws), [((m, n), F)],
+                    **plan)
+        return _bits(got).clone()
+
+    default, two = bits(), bits(gemm_small="0")
+    assert not torch.equal(default, two)
+    for value in ("", "default", "128,192", "96,96,3", "256,192,2,64,8"):
+        assert torch.equal(bits(gemm_pipe=value), default), value
+    assert torch.equal(bits(gemm_pipe="128,192,3,64"), two)
+    assert torch.equal(bits(gemm_pipe="0"), two)
+    assert torch.equal(bits(gemm_config="128,192,64,2,2,4"), two)
+    assert torch.equal(bits(gemm_config="96,96,64,2,2,4"), default)
+    assert torch.equal(bits(gemm_config="128,192,64,2,2,4", gemm_small="64,64,8,6,2"), default)
