@@ -1058,6 +1058,17 @@ double pipe_eff(const PipeConfig& c, Store st, Layout l) {
     return c.bm == 128 ? 0.80 : (c.bn == 256 ? 1.0 : 0.97);
 }
 
+// The k a configuration is charged for. A partial last step multiplies as a
+// whole one and loads only its part: in NT half of its padding counts (8192 x
+// 768, the 64-deep tail tile against 32-deep steps: k = 32 5.6 and 5.3 us, 160
+// 7.3 and 7.0, 352 10.1 and 10.0, 480 11.6 and 11.9, 800 15.9 and 16.7). In NN
+// the 64-deep steps' whole lines of x win at every k (k = 32 5.9 and 6.2 us, 160
+// 7.4 and 8.5, 480 11.6 and 14.5).
+double priced_k(const PipeConfig& c, Layout l, size_t k) {
+    const size_t whole = (k + c.bk - 1) / c.bk * c.bk;
+    return l == Layout::kNT ? 0.5 * (double(k) + double(whole)) : double(k);
+}
+
 // The macro-tile: whole waves of tiles over the CUs weigh most (a K = 768
 // tile is short, so a partial last wave costs nearly a full one); among equal
 // wave counts the larger tile needs fewer bytes per FLOP.
@@ -1087,7 +1098,8 @@ PipeConfig pick_pipe(size_t m, size_t n, size_t k, size_t slices, int cus, Store
         // output (8192 x 3072 x 768: 42.7 against 42.1 us for 128 x 192).
         if (c.loaders && c.bm == 256 && l != Layout::kTN && double(m) * double(n) < 1e8)
             continue;
-        const double cost = rounds * double(c.bm) * double(c.bn) / pipe_eff(c, st, l);
+        const double cost =
+            rounds * double(c.bm) * double(c.bn) * priced_k(c, l, k) / pipe_eff(c, st, l);
         if (cost < best_cost * 0.999) {
             best_cost = cost;
             best = c;
