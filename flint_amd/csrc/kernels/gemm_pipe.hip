@@ -996,13 +996,17 @@ size_t lds_bytes(const PipeConfig& c, Store st) {
 // The configuration with k-tail instances for NT and NN.
 bool has_tail(const PipeConfig& c) { return c.same(PipeConfig{128, 192, 3, 64}); }
 
+// k in whole k-steps (bk is a power of two: a division for each configuration
+// of each call showed in calls of a few us).
+size_t whole_k(const PipeConfig& c, size_t k) { return (k + c.bk - 1) & ~size_t(c.bk - 1); }
+
 // Whether a configuration can run an epilogue over k: it fits in LDS and k is
 // whole k-steps, or TN's FP32 output's, or the configuration takes tails (its
 // heads-view instances do not); the 8-wave configuration serves the NT layout
 // only.
 bool usable(const PipeConfig& c, Store st, size_t k, Layout l, bool views) {
     const bool tail = st == Store::kTn || (l != Layout::kTN && !views && has_tail(c));
-    return lds_bytes(c, st) <= kPipeMaxLds && (k % size_t(c.bk) == 0 || tail) &&
+    return lds_bytes(c, st) <= kPipeMaxLds && (whole_k(c, k) == k || tail) &&
            (c.waves == 4 || l == Layout::kNT);
 }
 
@@ -1065,8 +1069,7 @@ double pipe_eff(const PipeConfig& c, Store st, Layout l) {
 // the 64-deep steps' whole lines of x win at every k (k = 32 5.9 and 6.2 us, 160
 // 7.4 and 8.5, 480 11.6 and 14.5).
 double priced_k(const PipeConfig& c, Layout l, size_t k) {
-    const size_t whole = (k + c.bk - 1) / c.bk * c.bk;
-    return l == Layout::kNT ? 0.5 * (double(k) + double(whole)) : double(k);
+    return l == Layout::kNT ? 0.5 * (double(k) + double(whole_k(c, k))) : double(k);
 }
 
 // The macro-tile: whole waves of tiles over the CUs weigh most (a K = 768
@@ -1130,7 +1133,7 @@ void plan_tn(size_t m, size_t n, size_t k, int max_splits, int cus, bool accumul
         const double tiles = double((m + c.bm - 1) / c.bm) * double((n + c.bn - 1) / c.bn);
         for (int sp = 1; sp <= max_splits; ++sp) {
             const size_t len = (k + sp - 1) / sp;
-            const size_t len32 = (len + c.bk - 1) / c.bk * c.bk;
+            const size_t len32 = whole_k(c, len);
             if (size_t(sp - 1) * len32 >= k) continue;   // the last split would be empty
             const double rounds = std::ceil(tiles * sp / cus);
             // One 256 x 256 x 32 step of a unit is ~0.5 us at the pipeline's rate.
@@ -1175,7 +1178,7 @@ hipError_t launch_pipe(const PipeConfig& c, const Operands& op, size_t slices, i
     const dim3 grid(unsigned(gx), 1, 1);
     // Only the k-tail instances and TN's FP32 output have a partial last k-step:
     // any other would drop the k past the whole ones.
-    const bool whole = ST == Store::kTn || op.k % c.bk == 0;
+    const bool whole = ST == Store::kTn || whole_k(c, size_t(op.k)) == size_t(op.k);
 #define FLINT_PIPE_CASE(BM_, BN_, S_, BK_, NW_, LD_)                                           \
     if constexpr (pipe_lds_bytes<BM_, BN_, S_, BK_, L, ST, NW_>() <= kPipeMaxLds) {            \
         if (c.same(PipeConfig{BM_, BN_, S_, BK_, NW_, LD_})) {                                 \
@@ -1287,7 +1290,7 @@ hipError_t launch_gemm_pipe_tn(void* y, const void* x, const void* w, size_t m, 
     const bool force = pipe_forced(&forced, &disabled) && usable(forced, Store::kTn, k, Layout::kTN, false);
     plan_tn(m, n, k, workspace != nullptr ? max_splits : 1, cus, accumulate,
             force ? &forced : nullptr, &c, &sp);
-    const size_t len = ((k + sp - 1) / sp + c.bk - 1) / c.bk * c.bk;
+    const size_t len = whole_k(c, (k + sp - 1) / sp);
     Operands op{};
     op.y = y;
     op.x = static_cast<const _Float16*>(x);
@@ -1345,13 +1348,13 @@ bool gemm_pipe_override(GemmLayout gl, Epilogue e, size_t m, size_t n, size_t k,
 // where the rounds fill the GPU (the CUs then share the L2s and the power) and
 // where operand rows lie off the 128-byte lines, or are loaded half a line at
 // a time, so that each piece costs two lines. A round's prologue and epilogue
-// take 2.7 to 2.8 us, TN's FP32 output 4.6. The constants are fitted together with
+// take 2.7 to 2.8 us, TN's FP32 output 4.6; one round's GELU and residual
+// epilogues 2 us more, dGELU's 3. The constants are fitted together with
 // gemm_small.hip's.
-double gemm_pipe_estimate(GemmLayout gl, Epilogue e, size_t slices, size_t m, size_t n, size_t k,
-                          int max_splits, bool views) {
-    constexpr double kInfinite = 1e300;
+PipeEstimate gemm_pipe_estimate(GemmLayout gl, Epilogue e, size_t slices, size_t m, size_t n,
+                                size_t k, int max_splits, bool views) {
     int cus = 256;
-    if (!gemm_pipe_eligible(gl, e, m, n, k) || device_cus(&cus) != hipSuccess) return kInfinite;
+    if (!gemm_pipe_eligible(gl, e, m, n, k) || device_cus(&cus) != hipSuccess) return {};
     const Layout l = layout_of(gl);
     const Store st = store_of(e, l);
     PipeConfig c;
@@ -1360,19 +1363,30 @@ double gemm_pipe_estimate(GemmLayout gl, Epilogue e, size_t slices, size_t m, si
     else c = pick_pipe(m, n, k, slices, cus, st, l, views);
     const double tiles = double((m + c.bm - 1) / c.bm) * double((n + c.bn - 1) / c.bn) *
                          double(slices) * sp;
-    const double rounds = std::ceil(tiles / cus);
-    const double steps = double(k) / sp / 64.0;
+    const double load = tiles / cus, rounds = std::ceil(load);
+    const size_t len = (k + sp - 1) / sp;
+    const double steps = double(whole_k(c, len)) / 64.0;
     const bool off_lines = l == Layout::kTN ? m % 64 != 0 || n % 64 != 0 : k % 64 != 0 || c.bk == 32;
     const double layout = l == Layout::kNN ? 0.906 : 1.0;
     const double lines =
         !off_lines ? 1.0 : (l == Layout::kNN ? 1.53 : (l == Layout::kNT ? 1.34 : 1.5));
-    const double crowd = 1.0 + 1.38 * std::max(0.0, tiles / cus / rounds - 0.4);
+    const double crowd = 1.0 + 1.38 * std::max(0.0, load / rounds - 0.4);
     const double step_us = double(c.bm) * double(c.bn) / 65536.0 / pipe_eff(c, st, l) * layout *
                            lines * crowd;
     const double fixed = l == Layout::kTN ? 4.56 : (l == Layout::kNT ? 2.81 : 2.68);
-    double us = rounds * steps * step_us + fixed * (1.0 + 1.34 * (rounds - 1.0));
-    if (sp > 1) us += 3.0 + double(sp + 2) * double(m) * double(n) * 4.0 / 5e6;
-    return us;
+    const double epilogue = st == Store::kDGelu                                       ? 3.0
+                            : st == Store::kBiasGelu || st == Store::kBiasResidual ? 2.0
+                                                                                   : 0.0;
+    PipeEstimate out;
+    out.load = load;
+    out.us = rounds * steps * step_us + fixed * (1.0 + 1.34 * (rounds - 1.0));
+    if (sp > 1) out.us += 3.0 + double(sp + 2) * double(m) * double(n) * 4.0 / 5e6;
+    // Ragged k on less than half of the CUs, each streaming its strips in
+    // pieces that start anywhere in a line: NN 592 x 3512 x 2648 64.5 us, NT
+    // 865 x 2848 x 7672 193, twice what whole steps would take.
+    if (k % 32 != 0 && load < 0.5) out.us *= 1.4;
+    out.us += epilogue;
+    return out;
 }
 
 hipError_t launch_gemm_pipe(GemmLayout gl, Epilogue e, void* y, const void* x, const void* w,

@@ -54,9 +54,6 @@ namespace {
 
 constexpr int kStep = 64;   // k per step
 
-// gemm_pipe_estimate's value for a shape the pipeline does not take.
-constexpr double kNoEstimate = 1e300;
-
 // A split TN's sum of its partials: a launch of its own (us).
 constexpr double kSplitSumUs = 3.0;
 
@@ -484,6 +481,21 @@ constexpr SmallConfig kSmallConfigs[] = {
     {128, 64, 8, 3, 1, 2, {0.263, 0.347, 0.410}, {0.393, 0.499, 0.630}, {1.12, 0.198, 0.645}},
 };
 
+// The pipeline's workgroups store one tile while they load the next; here a
+// tile's stores are waited for before its CU's place is free. Over 1,050 drawn
+// products (16 to 16,384 rows, k from 8) the choice without this and the limit
+// below was slower than the kernel before by more than 3% for 65, up to 1.74
+// times, all of a round of pipeline tiles or more or of short k (TN 1472 x 50304 x 64
+// 61 -> 103 us, batched NT 38 x 640 x 640 x 64 10.9 -> 18.1); with them for 15, by
+// a tenth mostly.
+constexpr double kStoreMbPerUs = 6.0;
+constexpr double kMostPipeLoad = 1.25;
+
+// Bytes a product writes per output value.
+double out_bytes(Epilogue e) {
+    return e == Epilogue::kBiasGelu || e == Epilogue::kBiasResidual || e == kTnFloat ? 4.0 : 2.0;
+}
+
 int layout_index(GemmLayout l) { return l == GemmLayout::kNT ? 0 : (l == GemmLayout::kNN ? 1 : 2); }
 
 // Estimated us (past a launch's own) of `tiles` tiles of `steps` k-steps.
@@ -573,7 +585,12 @@ bool gemm_small_plan(GemmLayout l, Epilogue e, size_t slices, size_t m, size_t n
     if (!force && gemm_pipe_override(l, e, m, n, k, views)) return false;
     int cus = 256;
     if (device_cus(&cus) != hipSuccess) return false;
-    double best = force ? kNoEstimate : gemm_pipe_estimate(l, e, slices, m, n, k, max_splits, views);
+    const PipeEstimate pipe =
+        force ? PipeEstimate{} : gemm_pipe_estimate(l, e, slices, m, n, k, max_splits, views);
+    // From a round and a quarter of the pipeline's tiles on they are the faster
+    // ones, whatever the estimates say (kMostPipeLoad).
+    if (pipe.load > kMostPipeLoad) return false;
+    double best = pipe.us;
     // Ragged products the pipeline does not take would run gemm.hip's kernels:
     // slower up to about 60 rounds of 128 x 64 tiles (NT 2500 x 50257 x 768 465
     // against 446 us here; 6753 x 800 x 200 14.9 against 11.2), faster at 196
@@ -583,6 +600,7 @@ bool gemm_small_plan(GemmLayout l, Epilogue e, size_t slices, size_t m, size_t n
     // Only for a clear gain, so that no product gets slower by an estimate's
     // error (NN 1500 x 2272 x 568: 11.7 us here, 10.3 in the pipeline).
     if (best != kNoEstimate) best *= 0.9;
+    const double out_mb = double(slices) * double(m) * double(n) * out_bytes(e) / 1e6;
     bool taken = false;
     for (const SmallConfig& c : kSmallConfigs) {
         if (force && (c.bm != forced.bm || c.bn != forced.bn || c.waves != forced.waves)) continue;
@@ -592,6 +610,7 @@ bool gemm_small_plan(GemmLayout l, Epilogue e, size_t slices, size_t m, size_t n
             const size_t len = ((k + sp - 1) / sp + kStep - 1) / kStep * kStep;
             if (size_t(sp - 1) * len >= k || !fits_a_launch(tiles * sp, c.waves)) break;
             double cost = small_cost(c, l, tiles * sp, double(len / kStep), cus);
+            cost += double(sp) * out_mb / kStoreMbPerUs;
             if (sp > 1) cost += kSplitSumUs + double(sp + 2) * double(m) * double(n) * 4.0 / 5e6;
             if (cost < best) {
                 best = cost;

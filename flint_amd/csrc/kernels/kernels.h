@@ -48,10 +48,16 @@ hipError_t launch_gemm_pipe(GemmLayout l, Epilogue e, void* y, const void* x, co
                             hipStream_t stream, bool causal = false,
                             const HeadView* wv = nullptr, const HeadView* yv = nullptr);
 // The pipeline's estimated time for a product, us past a launch's own, with
-// the tile (and TN split, up to max_splits) it would choose; infinite where it
-// does not take the shape. views: the product reads and writes heads views.
-double gemm_pipe_estimate(GemmLayout l, Epilogue e, size_t slices, size_t m, size_t n, size_t k,
-                          int max_splits, bool views);
+// the tile (and TN split, up to max_splits) it would choose, and that tile's
+// count per CU; infinite where it does not take the shape. views: the product
+// reads and writes heads views.
+constexpr double kNoEstimate = 1e300;
+struct PipeEstimate {
+    double us = kNoEstimate;
+    double load = 0.0;
+};
+PipeEstimate gemm_pipe_estimate(GemmLayout l, Epilogue e, size_t slices, size_t m, size_t n,
+                                size_t k, int max_splits, bool views);
 // Whether the "gemm_pipe" override decides a product's kernel: it turns the
 // pipeline off, or names a tile that can run the product there.
 bool gemm_pipe_override(GemmLayout l, Epilogue e, size_t m, size_t n, size_t k, bool views);
