@@ -496,6 +496,25 @@ double out_bytes(Epilogue e) {
     return e == Epilogue::kBiasGelu || e == Epilogue::kBiasResidual || e == kTnFloat ? 4.0 : 2.0;
 }
 
+// Up to how many rounds of 128 x 64 tiles these kernels are faster than
+// gemm.hip's, which run what the pipeline does not take. Up to five: nearly
+// everywhere (NN 512 x 17000 x 65536, past 2^31 bytes, 3175 -> 2372 us; NT 64 x
+// 50301 x 7744 245 -> 183). Past that gemm.hip's larger tiles read less: TN 50304 x
+// 768 x 24576 2645 us against 4095, NN 24576 x 768 x 50304 2372 against 3316,
+// batched NT 96 x 1000 x 1000 x 520 231 against 278. Two exceptions: odd widths
+// (gemm.hip stores them value by value) while k is short (NT 8190 x 24001 x 768
+// 769 us and 646 here, x 1536 1035 and 1180; with bias 768 730 and 788; GELU's
+// second output moves the line to 2,048), and batched TN of ragged k (200 x 520 x
+// 520 x 520 672 and 188, 96 x 1000 x 1000 x 520 250 and 273). Either was measured
+// up to 96 rounds (NT 8192 x 50257 x 768, 196 of them: 1486 us and 1592).
+double most_rounds(GemmLayout l, Epilogue e, size_t n, size_t k) {
+    const size_t odd_k = e == Epilogue::kBiasGelu ? 2048
+                         : e == Epilogue::kNone || e == Epilogue::kScale ? 1280
+                                                                         : 640;
+    const bool batched_tn = l == GemmLayout::kTN && e == Epilogue::kNone;
+    return batched_tn || (n % 8 != 0 && k <= odd_k) ? 96.0 : 5.0;
+}
+
 int layout_index(GemmLayout l) { return l == GemmLayout::kNT ? 0 : (l == GemmLayout::kNN ? 1 : 2); }
 
 // Estimated us (past a launch's own) of `tiles` tiles of `steps` k-steps.
@@ -591,11 +610,8 @@ bool gemm_small_plan(GemmLayout l, Epilogue e, size_t slices, size_t m, size_t n
     // ones, whatever the estimates say (kMostPipeLoad).
     if (pipe.load > kMostPipeLoad) return false;
     double best = pipe.us;
-    // Ragged products the pipeline does not take would run gemm.hip's kernels:
-    // slower up to about 60 rounds of 128 x 64 tiles (NT 2500 x 50257 x 768 465
-    // against 446 us here; 6753 x 800 x 200 14.9 against 11.2), faster at 196
-    // (8192 x 50257 x 768 1486 against 1592).
-    if (best == kNoEstimate && !force && small_tiles(kSmallConfigs[4], slices, m, n) > 96.0 * cus)
+    if (best == kNoEstimate && !force &&
+        small_tiles(kSmallConfigs[4], slices, m, n) > most_rounds(l, e, n, k) * cus)
         return false;
     // Only for a clear gain, so that no product gets slower by an estimate's
     // error (NN 1500 x 2272 x 568: 11.7 us here, 10.3 in the pipeline).

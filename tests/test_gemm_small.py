@@ -198,6 +198,39 @@ def test_more_tiles_than_a_launch_holds(flint, cuda):
         assert torch.equal(y[r:r + 262140].float(), x[r:r + 262140].float() @ wt), r
 
 
+@pytest.mark.parametrize("plan", [{}, dict(gemm_small="0")], ids=["default", "general"])
+@pytest.mark.parametrize("layout", ["nt", "nn", "tn"])
+def test_an_operand_past_2_31_bytes(flint, cuda, layout, plan):
+    """Where the pipeline's 32-bit offsets end: few tiles run the few-tile
+    kernels, without them the general ones. Operands of -1, 0 and 1, so that
+    every sum is a whole number below 2,048 (six of its standard deviations,
+    171) and exact in FP32 and FP16 in any order."""
+    big, few, k = 16416, 64, 65536
+    g = torch.Generator(device=cuda).manual_seed(45)
+
+    def signs(*shape):
+        return torch.randint(-1, 2, shape, generator=g, device=cuda, dtype=H)
+
+    if layout == "nt":
+        x, w, m, n = signs(few, k), signs(big, k), few, big
+        call, out = lambda y: flint.gemm_nt(y, x, w, m, n, k), H
+    elif layout == "nn":
+        x, w, m, n = signs(few, k), signs(k, big), few, big
+        call, out = lambda y: flint.gemm_nn(y, x, w, m, n, k), H
+    else:
+        x, w, m, n = signs(k, big), signs(k, few), big, few
+        ws = torch.empty(flint.gemm_tn_workspace(m, n, k), dtype=torch.uint8, device=cuda)
+        call, out = lambda y: flint.gemm_tn(y, x, w, m, n, k, workspace=ws), F
+    got, = _run(flint, call, [((m, n), out)], **plan)
+    ref = torch.zeros(m, n, device=cuda)
+    for c in range(0, k, 4096):
+        xs = x[c:c + 4096].t() if layout == "tn" else x[:, c:c + 4096]
+        ws_ = w[:, c:c + 4096].t() if layout == "nt" else w[c:c + 4096]
+        ref += xs.float().contiguous() @ ws_.float().contiguous()
+    assert float(ref.abs().max()) < 2048
+    assert torch.equal(got.float(), ref)
+
+
 def test_which_overrides_decide_the_kernel(flint, cuda):
     """TN 768 x 768 x 3000 shows its plan in its bits: by default the few-tile
     kernels sum k in one piece, the pipeline and the general kernel in two of
