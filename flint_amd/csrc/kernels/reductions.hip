@@ -307,8 +307,8 @@ __device__ __forceinline__ float merge_few_chunks(const ChunkColumns<COLS>& sums
 // column_finish's merge of them from LDS. What bounds it is latency, of one
 // round of loads and of the sums' chain; the second launch for a few KB of
 // partials cost as much again. One MI355X, launches included: 256 x 768 7.1 ->
-// 4.0 us, 512 x 2304 7.2 -> 4.7, 1000 x 800 7.3 -> 4.8, 2048 x 768 7.2 -> 6.7;
-// 2048 x 3072, whose bytes count, 8.7 -> 11.1 (two launches there). Two layers'
+// 4.0 us, 512 x 2304 7.2 -> 4.7, 1000 x 800 7.3 -> 4.8, 2048 x 768 7.2 -> 6.7
+// (bias_gradient_one_launch has the line). Two layers'
 // gradients of as many rows share a launch where a caller has both at hand, as
 // neither fills the GPU (GPT-2's training step on 256 tokens, 48 of them:
 // 2,360 -> 2,256 us).
@@ -1023,10 +1023,14 @@ hipError_t launch_params_merge(const ParamsMerge& merge, hipStream_t stream) {
 }
 
 bool bias_gradient_one_launch(size_t rows, size_t cols) {
-    // Measured even at 1024 x 3072 (7.1 against 7.5 us), see bias_gradient_few.
-    constexpr size_t kMostValues = size_t{4} << 20;
-    return rows <= size_t(kFewChunks) * kChunkRows && rows * cols <= kMostValues &&
-           !tuning_off(Tune::kSumsFew);
+    // Even with two launches at 512 x 8192 at least (6.0 against 8.1 us there),
+    // 1024 x 3072 (7.9 and 7.9; x 4096 9.0 and 8.1), 1536 x 1600 (6.3 and 7.4; x
+    // 2048 8.7 and 7.9) and 2048 x 768 (6.8 and 7.3; x 1024 7.6 and 7.2, x 2048 10.6
+    // and 8.4): the values count, and from three chunks on, where workgroups hold
+    // 16 columns, a wave's chain of rows as well.
+    if (rows > size_t(kFewChunks) * kChunkRows || tuning_off(Tune::kSumsFew)) return false;
+    if (rows <= 2 * kChunkRows) return rows * cols <= size_t{4} << 20;
+    return rows * cols <= 3200000 && rows * rows * cols <= size_t{3800000000};
 }
 
 hipError_t launch_bias_gradients_few(const BiasGradient& one, const BiasGradient& two, size_t rows,

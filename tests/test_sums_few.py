@@ -1,5 +1,5 @@
 """Column sums of few 256-row chunks finished in their own launch: the bias
-gradient (up to 8 chunks) and LayerNorm backward's dbeta and dgamma (up to 4),
+gradient (up to 8 chunks) and LayerNorm backward's dbeta and dgamma (one),
 at the chunk counts where the plans change and past them, bit for bit against
 the C oracle, with infinities, NaN and -0 among the values."""
 
@@ -36,6 +36,24 @@ def test_bias_gradient(flint, cuda, rows, cols):
         torch.cuda.synchronize()
         ref = oracle.bias_gradient(dy.numpy(), old.numpy() if accumulate else None)
         assert np.array_equal(_bits(out), _bits(ref))
+
+
+# Either side of each line of bias_gradient_one_launch.
+@pytest.mark.parametrize("rows,cols", [(512, 8192), (512, 8200), (513, 6232), (513, 6240),
+                                       (1024, 3120), (1024, 3128), (1536, 1608), (1536, 1616),
+                                       (2048, 904), (2048, 912)])
+def test_bias_gradient_where_the_plan_changes(flint, cuda, tune, rows, cols):
+    dy = normal((rows, cols), rows, 1.0, torch.float16).to(cuda)
+
+    def run():
+        out = normal((cols,), 7).to(cuda)
+        flint.bias_gradient(out, dy, rows, cols, accumulate=True)
+        torch.cuda.synchronize()
+        return out
+
+    got = run()
+    tune("sums_few", "0")
+    assert np.array_equal(_bits(got), _bits(run()))
 
 
 @pytest.mark.parametrize("rows", [1, 256, 257, 1000, 1024, 1025])
