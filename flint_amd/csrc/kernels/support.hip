@@ -543,6 +543,7 @@ column_sums_one_chunk(float* __restrict__ out, const float* __restrict__ dy, int
 constexpr int kScanRows = 8192;   // tokens embedding_scan_runs holds in LDS
 constexpr int kScanWaves = 8;     // positions (one a wave) per workgroup
 constexpr int kScanThreads = kScanWaves * 64;
+constexpr int kScanFewBlocks = 256;   // workgroups that few positions are spread over
 constexpr int kScanBlock = 512;   // positions a wave tests at a time, 8 a lane
 constexpr int kScanBlocks = kScanRows / kScanBlock;
 constexpr int kScanBatch = 4;     // rows of a short run whose loads go out together
@@ -581,26 +582,29 @@ struct BlockMatches {
         for (int k = 0; k < 8; ++k) n += __builtin_popcountll(m[k]);
         return n;
     }
-    // The first of them (any() != 0).
-    __device__ __forceinline__ int first(int base) const {
-        const int l = __builtin_ctzll(any());
-        unsigned at = 0;   // bit k: position k of lane l (no index into m: it stays in registers)
+    // Whether one of them is below base + at (at < 512).
+    __device__ __forceinline__ bool below(int at) const {
+        const int l = at >> 3;
+        if ((any() & ((uint64_t{1} << l) - 1)) != 0) return true;
+        bool found = false;   // in lane l (no index into m: it stays in registers)
 #pragma unroll
-        for (int k = 0; k < 8; ++k) at |= unsigned((m[k] >> l) & 1) << k;
-        return base + 8 * l + __builtin_ctz(at);
+        for (int k = 0; k < 7; ++k) found |= k < (at & 7) && ((m[k] >> l) & 1) != 0;
+        return found;
     }
     // Writes them in ascending order to list[at], list[at + 1], ...: a lane's
     // rank is the matches of the lanes below it. Entries from `cap` on are
     // left out.
     __device__ __forceinline__ void append(uint16_t* list, int at, int cap, int base, int lane) const {
-        const uint64_t below = (uint64_t{1} << lane) - 1;
-        int rank = at;
+        unsigned rank = unsigned(at);
 #pragma unroll
-        for (int k = 0; k < 8; ++k) rank += __builtin_popcountll(m[k] & below);
+        for (int k = 0; k < 8; ++k)
+            rank = __builtin_amdgcn_mbcnt_hi(unsigned(m[k] >> 32),
+                                             __builtin_amdgcn_mbcnt_lo(unsigned(m[k]), rank));
 #pragma unroll
         for (int k = 0; k < 8; ++k) {
+            if (m[k] == 0) continue;   // the same for the wave: few of the eight hold a match
             if ((m[k] >> lane) & 1) {
-                if (rank < cap) list[rank] = uint16_t(base + 8 * lane + k);
+                if (rank < unsigned(cap)) list[rank] = uint16_t(base + 8 * lane + k);
                 ++rank;
             }
         }
@@ -628,10 +632,13 @@ __device__ __forceinline__ float run_value(float old, const Comp& s) {
 //    or two columns, 16 rows' loads in flight while 16 are added.
 // Text has few frequent words and they all start near the front: positions
 // are dealt to workgroups a grid apart, so that their runs spread over the
-// GPU. At 8 x 1024 x 768 (one MI355X, position sums included): text-like
-// tokens (257 rows of the most frequent) 114.5 -> 27.1 us against one wave a
-// run at every length,
-// uniform ones 23.0 -> 24.1, Zipf s = 1.1 (a run of 1,113) 441 -> 77.
+// GPU; with few of them, one or two to a workgroup. One MI355X, position sums
+// included, against one wave a run at every length and four positions a
+// workgroup: 8 x 1024 x 768 text-like tokens (257 rows of the most frequent)
+// 114.5 -> 27.1 us, Zipf s = 1.1 (a run of 1,113) 477 -> 81, uniform ones 22.7 ->
+// 23.3; 1 x 256 x 768 uniform ones 3.5 -> 3.5, x 256 2.65 -> 2.95. What short runs
+// pay for it: a barrier, and their list through LDS (4 x 1024 x 256, every token
+// twice in a row, 5.6 -> 7.7).
 // Workgroups from run_blocks on take column quads of the position gradient
 // (column_sums_quad, as in sort_tokens_and_positions).
 template <int G>
@@ -670,16 +677,22 @@ embedding_scan_runs(float* __restrict__ dwte, const float* __restrict__ dx,
             BlockMatches bm;
             bm.test(t, base, rows, v, lane);
             if (bm.any() == 0) continue;
-            if (n == 0 && bm.first(base) < i) break;   // an earlier position's run
-            if (n < kScanShort) bm.append(shorts[wave], n, kScanShort, base, lane);
-            n += bm.count();
+            if (n == 0 && (base + kScanBlock <= i || bm.below(i - base))) break;   // an earlier one's run
+            const int here = bm.count();
+            // A run of one row needs no list, a later row puts it there.
+            if (n + here > 1 && n < kScanShort) {
+                if (n == 1 && lane == 0) shorts[wave][0] = uint16_t(i);
+                bm.append(shorts[wave], n, kScanShort, base, lane);
+            }
+            n += here;
         }
     }
     if (lane == 0) runs[wave] = n > kScanShort ? n : 0;
     if (n > 0 && n <= kScanShort) {
-        // Other lanes wrote the list.
+        // Other lanes wrote the list. Lane u holds its entry u.
         __builtin_amdgcn_wave_barrier();
         asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        const int list = n == 1 ? i : int(shorts[wave][lane & (kScanShort - 1)]);
         float* const out = dwte + size_t(tok[i]) * width;
         const size_t col0 = size_t(lane) * 4;
         Comp s[G][4];
@@ -694,7 +707,7 @@ embedding_scan_runs(float* __restrict__ dwte, const float* __restrict__ dx,
 #pragma unroll
             for (int u = 0; u < kScanBatch; ++u) {
                 const bool live = k + u < n;
-                const size_t row = live ? size_t(__builtin_amdgcn_readfirstlane(int(shorts[wave][k + u]))) : 0;
+                const size_t row = live ? size_t(__builtin_amdgcn_readlane(list, k + u)) : 0;
 #pragma unroll
                 for (int g = 0; g < G; ++g) {
                     const size_t col = col0 + size_t(g) * 256;
@@ -723,9 +736,12 @@ embedding_scan_runs(float* __restrict__ dwte, const float* __restrict__ dx,
         }
     }
     __syncthreads();
-    for (int owner = 0; owner < kScanWaves; ++owner) {
-        const int total = runs[owner];
-        if (total == 0) continue;   // the same for every thread
+    // The long runs, one by one (mostly none).
+    const int long_runs = runs[lane & (kScanWaves - 1)];
+    uint64_t owners = __builtin_amdgcn_ballot_w64(long_runs != 0) & ((1u << kScanWaves) - 1);
+    for (; owners != 0; owners &= owners - 1) {   // the same for every thread
+        const int owner = __builtin_ctzll(owners);
+        const int total = __builtin_amdgcn_readlane(long_runs, owner);
         const uint16_t v = tok[owner * int(run_blocks) + int(blockIdx.x)];
         // List the run's rows: the blocks' counts, then each block's rows
         // after those of the blocks before it.
@@ -968,7 +984,10 @@ hipError_t launch_embedding_backward(void* dwte, void* dwpe, const void* dx, con
     // Accumulating into dwte, with the tokens in one workgroup's LDS: the
     // token rows without a sort ("emb_scan" = "0": the sorted path).
     const size_t groups = (width + 255) / 256;
-    const size_t run_blocks = (rows + kScanWaves - 1) / kScanWaves;
+    // Few positions go to a wave in as many workgroups as there are CUs: eight
+    // to a workgroup, 16 to 1,000 of them took 1.0 us longer.
+    const size_t run_blocks =
+        std::max((rows + kScanWaves - 1) / kScanWaves, std::min<size_t>(rows, kScanFewBlocks));
     if (accumulate_wte && rows <= size_t(kScanRows) && groups <= 4 &&
         run_blocks + scan_pos_blocks < (size_t{1} << 31) && !tuning_off(Tune::kEmbScan)) {
         const dim3 grid(unsigned(run_blocks + scan_pos_blocks));

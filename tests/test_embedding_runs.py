@@ -18,8 +18,21 @@ RUNS = [1, 4, 5, 15, 16, 17, 31, 32, 33, 47, 48, 49, 63, 64, 65, 129]
 
 @pytest.mark.parametrize("width", [8, 256, 264, 520, 768, 1000])
 def test_runs_of_every_length(flint, cuda, width):
-    vocab = len(RUNS) + 3
-    tok = torch.cat([torch.full((n,), v, dtype=torch.int64) for v, n in enumerate(RUNS)])
+    _check(flint, cuda, RUNS, width)
+
+
+@pytest.mark.parametrize("width", [8, 264, 768])
+@pytest.mark.parametrize("rows", [2000, 2600, 8192])
+def test_short_runs_over_many_workgroups(flint, cuda, width, rows):
+    """Beside the long runs mostly pairs, whose rows lie blocks apart, and
+    single rows; more positions than workgroups, up to the most tokens."""
+    left = rows - sum(RUNS)
+    _check(flint, cuda, RUNS + [2] * (left // 4) + [1] * (left - left // 4 * 2), width)
+
+
+def _check(flint, cuda, runs, width):
+    vocab = len(runs) + 3
+    tok = torch.cat([torch.full((n,), v, dtype=torch.int64) for v, n in enumerate(runs)])
     tok = tok[torch.randperm(len(tok), generator=torch.Generator().manual_seed(width))]
     sequences, length = 1, len(tok)
     dx = normal((length, width), 21)
