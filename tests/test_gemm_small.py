@@ -1,9 +1,10 @@
 """The few-tile GEMM kernels (gemm_small.hip), each configuration forced: every
 layout and epilogue at edges of tiles, k tails and odd widths, bit for bit
 against the other kernels (one MFMA chain over k either way), inside guard
-bands. TN's FP32 output may split k elsewhere, so it is held to float32 sums in
-another order: |difference| <= 2 k eps sum |x w|, far above what any order
-gives and far below a missing or doubled product."""
+bands. TN's FP32 output may split k elsewhere from k = 2048 on: below it is held
+to the bits as well, and whole-number operands, whose sums are exact in any
+order, show a missing or doubled product at every k. Beside that it stays within
+2 k eps sum |x w| of float64."""
 
 import pytest
 import torch
@@ -102,6 +103,11 @@ def test_tn(flint, cuda, cfg, m, n, k, accumulate):
     ref = x.double().t() @ w.double() + (y0.double() if accumulate else 0)
     bound = 2 * k * 2.0 ** -24 * (x.double().abs().t() @ w.double().abs()) + 2.0 ** -22 * ref.abs()
     assert bool(((got.double() - ref).abs() <= bound).all())
+    if k < 2048:
+        _same(flint, "one piece", call, [((m, n), F)], cfg)
+    x, w, y0 = (x * 20).round(), (w * 4).round(), (y0 * 4).round()
+    got, = _run(flint, call, [((m, n), F)], gemm_small=cfg)
+    assert torch.equal(got.double(), x.double().t() @ w.double() + (y0.double() if accumulate else 0))
 
 
 @pytest.mark.parametrize("cfg", CONFIGS)
@@ -175,11 +181,20 @@ def test_pipeline_tn_takes_any_k(flint, cuda, cfg, m, n, k):
     x = normal((k, m), 36, 0.1, H).to(cuda)
     w = uniform((k, n), 37).to(cuda)
     ws = torch.empty(max(flint.gemm_tn_workspace(m, n, k), 16), dtype=torch.uint8, device=cuda)
-    got, = _run(flint, lambda y: flint.gemm_tn(y, x, w, m, n, k, workspace=ws), [((m, n), F)],
-                gemm_pipe=cfg, gemm_small="0")
+    def call(y):
+        flint.gemm_tn(y, x, w, m, n, k, workspace=ws)
+
+    plan = dict(gemm_pipe=cfg, gemm_small="0")
+    got, = _run(flint, call, [((m, n), F)], **plan)
     ref = x.double().t() @ w.double()
     bound = 2 * k * 2.0 ** -24 * (x.double().abs().t() @ w.double().abs()) + 2.0 ** -22 * ref.abs()
     assert bool(((got.double() - ref).abs() <= bound).all())
+    if k < 2048:   # one piece
+        few, = _run(flint, call, [((m, n), F)], gemm_small="64,64,4,4,1")
+        assert torch.equal(_bits(got), _bits(few))
+    x, w = (x * 20).round(), (w * 4).round()   # exact sums in any order
+    got, = _run(flint, call, [((m, n), F)], **plan)
+    assert torch.equal(got.double(), x.double().t() @ w.double())
 
 
 def test_more_tiles_than_a_launch_holds(flint, cuda):
