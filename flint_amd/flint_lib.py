@@ -151,11 +151,12 @@ def stream_handle(stream):
     return stream.cuda_stream
 
 
-def _current_stream():
+def _first_current_stream():
     """torch's current stream on the calling thread, as a handle. Asked of torch
     directly: torch.cuda.current_stream() builds a Stream object, 3.0 us of a
     call's 7.4 (this way 0.2 us, a call 4.7). It also initialises torch's HIP
-    state, so the first call here goes through it."""
+    state, or says that this process cannot (a fork of one that did), so the
+    first call of a process goes through it."""
     global _current_stream
     import torch
 
@@ -165,6 +166,17 @@ def _current_stream():
     if device is not None and raw is not None:
         _current_stream = lambda: raw(device())  # noqa: E731
     return handle
+
+
+_current_stream = _first_current_stream
+
+
+def _after_fork():
+    global _current_stream
+    _current_stream = _first_current_stream
+
+
+os.register_at_fork(after_in_child=_after_fork)
 
 
 def library_path():
