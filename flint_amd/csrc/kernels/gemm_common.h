@@ -1,6 +1,6 @@
 // Definitions shared by the GEMM kernels (gemm.hip: the register-staged and
-// two-workgroup-per-CU family; gemm_pipe.hip: the one-wave-per-SIMD NT
-// pipeline): vector types, the epilogue kinds, the LDS swizzle, GELU and its
+// two-workgroup-per-CU family; gemm_pipe.hip: the one-wave-per-SIMD pipeline;
+// gemm_small.hip: products of few tiles): vector types, the epilogue kinds, the LDS swizzle, GELU and its
 // derivative, the tile map, wait and barrier helpers, and the kernel operands.
 #pragma once
 
@@ -167,10 +167,10 @@ struct Operands {
     float scale;
     int accumulate;        // TN: y += instead of y =
     int m, n, k;
-    int causal;            // attention (pipeline only): the per-slice m x m
+    int causal;            // attention (not gemm.hip): the per-slice m x m
                            // operand (NT's y, NN's and TN's x) is zero, or
                            // not wanted, above its diagonal
-    HeadView wv, yv;       // batched NN / TN (pipeline only): w (k-major) and
+    HeadView wv, yv;       // batched NN / TN (not gemm.hip): w (k-major) and
                            // y as heads views
 };
 

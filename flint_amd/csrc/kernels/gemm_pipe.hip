@@ -1,8 +1,9 @@
 // The GEMM pipeline on gfx950 with one wave per SIMD and large wave tiles,
 // for all three layouts (NT, NN, TN, and their batched forms) where rows of
 // operands and output are 16-byte multiples (TN's FP32 output: any k; batched
-// products: k a multiple of 32). Products of few tiles and most ragged ones
-// run gemm_small.hip's kernels, what is left gemm.hip's.
+// NT and TN: k a multiple of 32) and below 2^31 bytes. Products of few tiles run
+// gemm_small.hip's kernels (gemm_small_plan), ragged and larger ones those or
+// gemm.hip's.
 //
 // Why this shape of kernel (measured on MI355X):
 //  * A CU's L2 -> LDS rate depends on the row piece one load covers: 64-byte
@@ -1313,8 +1314,9 @@ bool gemm_pipe_eligible(GemmLayout gl, Epilogue e, size_t m, size_t n, size_t k)
     const Layout l = layout_of(gl);
     const Store st = store_of(e, l);
     // NT and NN take k tails in whole 16-byte chunks; TN's FP32 output any k.
-    // The batched forms keep to whole 32-deep steps, which the GPT-2 model's
-    // attention layout (heads views, causal spans) is planned on.
+    // Batched NT and TN keep to whole 32-deep steps, and with TN so does the GPT-2
+    // model's attention layout (heads views, causal spans); batched NN, whose
+    // slices are NN products, takes their tails.
     const bool batched = st == Store::kScale || st == Store::kTnHalf;
     if (batched ? k % kPipeBK != 0 : (l != Layout::kTN && k % 8 != 0)) return false;
     // Only the epilogues each layout serves.

@@ -1,4 +1,4 @@
-// GEMMs whose output has few tiles: 64 x 64 and 32 x 32 tiles, one per
+// GEMMs whose output has few tiles: tiles of 32 x 32 to 128 x 64, one per
 // workgroup, for every layout, epilogue and size the entry points take.
 //
 // A product with a few hundred rows leaves gemm_pipe.hip's 128 x 192 tiles on
@@ -457,11 +457,12 @@ __global__ void __launch_bounds__(NW * 64) gemm_small(Operands op, TileArgs ta) 
 // A configuration and its cost in us: `alone` is a k-step of a tile that has
 // its CU to itself, `shared` a tile's k-step where the CU runs several, `fixed`
 // a tile's prologue and epilogue. Each per layout NT, NN, TN (FP32 stores).
-// Fitted, together with gemm_pipe_estimate's constants, to the measured times
-// of 270 products (16 to 8,192 rows, widths 64 to 50,304, k 16 to 50,304,
-// batched ones among them; one MI355X, operands rotated past the caches): the
-// kernel and tile that the estimates choose are within 7% of the fastest for
-// all but 10 of them, at worst 1.3 times it.
+// Fitted, together with gemm_pipe_estimate's constants, to measured times of
+// products of 16 to 8,192 rows, widths 64 to 50,304 and k 16 to 50,304, batched
+// ones among them (one MI355X, operands rotated past the caches). Of 1,047 drawn
+// ones timed on every kernel and tile, the choice (with the charges and limits
+// below) is within 7% of the fastest for 929, at worst 1.65 times it, 2.6% in the
+// geometric mean.
 struct SmallConfig {
     int bm, bn, waves, stages, unit;
     int resident;   // workgroups a CU holds
@@ -486,8 +487,10 @@ constexpr SmallConfig kSmallConfigs[] = {
 // products (16 to 16,384 rows, k from 8) the choice without this and the limit
 // below was slower than the kernel before by more than 3% for 65, up to 1.74
 // times, all of a round of pipeline tiles or more or of short k (TN 1472 x 50304 x 64
-// 61 -> 103 us, batched NT 38 x 640 x 640 x 64 10.9 -> 18.1); with them for 15, by
-// a tenth mostly.
+// 61 -> 103 us, batched NT 38 x 640 x 640 x 64 10.9 -> 18.1); with them for 17, ten
+// of them of ragged k, where gemm.hip's kernels now and then are the fastest (NT +
+// residual 1391 x 1536 x 5192 71 us and 90; in the geometric mean over ragged k the
+// choice takes 0.55 of their time).
 constexpr double kStoreMbPerUs = 6.0;
 constexpr double kMostPipeLoad = 1.25;
 

@@ -24,9 +24,10 @@ enum class Epilogue { kNone, kBias, kBiasGelu, kBiasResidual, kDGelu, kScale };
 hipError_t launch_gemm_nt(void* y, const void* x, const void* w, const void* bias,
                           void* aux, Epilogue e, size_t m, size_t n, size_t k,
                           hipStream_t stream);
-// The one-wave-per-SIMD GEMM pipeline (gemm_pipe.hip), for k % 32 == 0 and
-// n % 8 == 0 (and m % 8 == 0 for TN). The launchers below route there when
-// gemm_pipe_eligible says so (FLINT_GEMM_PIPE=0 turns it off).
+// The one-wave-per-SIMD GEMM pipeline (gemm_pipe.hip), for n % 8 == 0 (and m %
+// 8 == 0 for TN), k % 8 == 0 (TN's FP32 output any k, batched NT and TN k % 32
+// == 0) and operands and outputs below 2^31 bytes: gemm_pipe_eligible (the
+// "gemm_pipe" override "0" turns it off).
 enum class GemmLayout { kNT, kNN, kTN };
 // kTnFloat: TN's FP32 output (y = sum, y += sum, or a split's partial);
 // kNone with TN is the batched FP16 output.
@@ -109,9 +110,9 @@ __host__ __device__ inline size_t head_view_offset(const HeadView& v, int slice)
 
 // The batched GEMMs. causal (attention inside the GPT-2 model only): x (NN,
 // TN) is zero above its diagonal per slice, or (NT) only y's entries at or
-// below the diagonal are wanted; the pipeline then skips the rest, which
-// changes no wanted value (the skipped products are exact zeros). Shapes the
-// pipeline does not take compute everything.
+// below the diagonal are wanted; the pipeline and the few-tile kernels then
+// skip the rest, which changes no wanted value (the skipped products are exact
+// zeros). gemm.hip's kernels compute everything.
 hipError_t launch_gemm_nt_batched(void* y, const void* x, const void* w, size_t batches,
                                   size_t m, size_t n, size_t k, float scale, hipStream_t stream,
                                   bool causal = false);
