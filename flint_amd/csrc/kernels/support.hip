@@ -636,7 +636,7 @@ __device__ __forceinline__ float run_value(float old, const Comp& s) {
 // included, against one wave a run at every length and four positions a
 // workgroup: 8 x 1024 x 768 text-like tokens (257 rows of the most frequent)
 // 114.5 -> 27.1 us, Zipf s = 1.1 (a run of 1,113) 477 -> 81, uniform ones 22.7 ->
-// 23.3; 1 x 256 x 768 uniform ones 3.5 -> 3.5, x 256 2.65 -> 2.95. What short runs
+// 23.2; 1 x 256 x 768 uniform ones 3.5 -> 3.3, x 256 2.65 -> 2.95. What short runs
 // pay for it: a barrier, and their list through LDS (4 x 1024 x 256, every token
 // twice in a row, 5.6 -> 7.7).
 // Workgroups from run_blocks on take column quads of the position gradient
