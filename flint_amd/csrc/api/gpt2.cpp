@@ -656,7 +656,7 @@ flint_status linear_grads(const flint_gpt2& m, const Param& w, const Param& b, c
                                                 m.tn_work, &splits, hs));
     // Few rows: the weight gradient unsplit and the bias gradient in a launch
     // of its own leave the finish nothing to do.
-    if (splits == 1 && flint::bias_gradient_one_launch(m.rows, b.cols)) {
+    if (splits == 1 && flint::bias_gradient_one_launch(m.rows, b.cols, true)) {
         const flint::BiasGradient bias{b.grad, dy, b.cols, acc != 0};
         if (pair) m.pending_bias = bias;
         else FLINT_TRY(flush_bias(m, bias, st));

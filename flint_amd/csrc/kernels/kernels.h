@@ -218,8 +218,9 @@ hipError_t launch_layernorm_backward(void* dx, void* dgamma, void* dbeta, const 
 hipError_t launch_params_merge(const ParamsMerge& merge, hipStream_t stream);
 hipError_t launch_bias_gradient(void* dbias, const void* dy, size_t rows, size_t cols,
                                 bool accumulate, void* workspace, hipStream_t stream);
-// Whether launch_bias_gradient takes this shape in one launch (no workspace).
-bool bias_gradient_one_launch(size_t rows, size_t cols);
+// Whether a bias gradient of this shape takes one launch (no workspace): by
+// itself, as launch_bias_gradient runs it, or in a training step (in_step).
+bool bias_gradient_one_launch(size_t rows, size_t cols, bool in_step);
 // Two bias gradients over the same number of rows that each take one launch
 // (bias_gradient_one_launch), in one; an empty one (cols 0) is none.
 struct BiasGradient {

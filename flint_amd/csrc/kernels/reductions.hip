@@ -1029,14 +1029,18 @@ hipError_t launch_params_merge(const ParamsMerge& merge, hipStream_t stream) {
     return hipGetLastError();
 }
 
-bool bias_gradient_one_launch(size_t rows, size_t cols) {
+bool bias_gradient_one_launch(size_t rows, size_t cols, bool in_step) {
     // Even with two launches at 512 x 8192 at least (6.0 against 8.1 us there),
     // 1024 x 3072 (7.9 and 7.9; x 4096 9.0 and 8.1), 1536 x 1600 (6.3 and 7.4; x
     // 2048 8.7 and 7.9) and 2048 x 768 (6.8 and 7.3; x 1024 7.6 and 7.2, x 2048 10.6
     // and 8.4): the values count, and from three chunks on, where workgroups hold
     // 16 columns, a wave's chain of rows as well.
     if (rows > size_t(kFewChunks) * kChunkRows || tuning_off(Tune::kSumsFew)) return false;
-    if (rows <= 2 * kChunkRows) return rows * cols <= size_t{4} << 20;
+    // A training step's two launches are the weight gradient's finish, which it
+    // has none of here, and a partials launch; and its one launch may carry
+    // another layer's sums (8 x 256 tokens, width 256, two layers: 399 us with
+    // this line, 411 with the one below).
+    if (in_step || rows <= 2 * kChunkRows) return rows * cols <= size_t{4} << 20;
     return rows * cols <= 3200000 && rows * rows * cols <= size_t{3800000000};
 }
 
@@ -1060,7 +1064,7 @@ hipError_t launch_bias_gradients_few(const BiasGradient& one, const BiasGradient
 
 hipError_t launch_bias_gradient(void* dbias, const void* dy, size_t rows, size_t cols,
                                 bool accumulate, void* workspace, hipStream_t stream) {
-    if (bias_gradient_one_launch(rows, cols))
+    if (bias_gradient_one_launch(rows, cols, false))
         return launch_bias_gradients_few({dbias, dy, cols, accumulate}, {}, rows, stream);
     if (hipError_t e = launch_partials(static_cast<float*>(workspace), dy, rows, cols, stream);
         e != hipSuccess) {
